@@ -1126,25 +1126,39 @@ __global__ void k_marginals(const float* __restrict__ B, float* __restrict__ A, 
   if (i < n) A[i] = marginal(B[i]);
 }
 
-// max |marginal(B) - Aprev| as an IEEE double reduced through the ordered bit
-// pattern of non-negative doubles; Aprev is refreshed in the same sweep.
-__global__ __launch_bounds__(256) void k_residual(const float* __restrict__ B, float* __restrict__ A, size_t n,
-                                                   unsigned long long* __restrict__ d_max) {
-  __shared__ double sh[256];
-  double m = 0.0;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const float a = marginal(B[i]);
-    const double dlt = fabs((double)a - (double)A[i]);
-    A[i] = a;
-    m = dlt > m ? dlt : m;
-  }
-  sh[threadIdx.x] = m;
+// max over the block's threads of m (>= 0) into *d_max through the ordered
+// bit pattern of non-negative doubles: one atomic per block, none when it
+// would not raise the maximum read before it (the atomics of a launch all go
+// to one word, and thousands of them take longer than the sweep of a small map)
+__device__ __forceinline__ void block_max(double m, unsigned long long* __restrict__ d_max) {
+  __shared__ double sh[4];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63u) == 0u) sh[threadIdx.x >> 6] = m;
   __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + off]);
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    m = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+    if (bits > __hip_atomic_load(d_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(d_max, bits);
   }
-  if (threadIdx.x == 0) atomicMax(d_max, (unsigned long long)__double_as_longlong(sh[0]));
+}
+
+// max |marginal(B) - Aprev| as an IEEE double; Aprev is refreshed in the same
+// sweep (stored only where it changes: most voxels are saturated and keep
+// their bits, so a third of the traffic is left out).  n is a multiple of 4.
+__global__ __launch_bounds__(256) void k_residual(const float4* __restrict__ B, float4* __restrict__ A, size_t n4,
+                                                   unsigned long long* __restrict__ d_max) {
+  double m = 0.0;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
+    const float4 b = B[i], p = A[i];
+    const float4 a = make_float4(marginal(b.x), marginal(b.y), marginal(b.z), marginal(b.w));
+    const double dx = fabs((double)a.x - (double)p.x), dy = fabs((double)a.y - (double)p.y);
+    const double dz = fabs((double)a.z - (double)p.z), dw = fabs((double)a.w - (double)p.w);
+    const double d = fmax(fmax(dx, dy), fmax(dz, dw));
+    if (!(d == 0.0)) A[i] = a;
+    m = fmax(m, d);
+  }
+  block_max(m, d_max);
 }
 
 // max |alpha(v) - ref(v)| with alpha the readback marginal (A, or 0 where
@@ -1152,20 +1166,13 @@ __global__ __launch_bounds__(256) void k_residual(const float* __restrict__ B, f
 __global__ __launch_bounds__(256) void k_ref_error(const float* __restrict__ A, const uint8_t* __restrict__ upd,
                                                    const float* __restrict__ ref, size_t n,
                                                    unsigned long long* __restrict__ d_max) {
-  __shared__ double sh[256];
   double m = 0.0;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
     const float a = upd[i] ? A[i] : 0.0f;
     const double dlt = fabs((double)a - (double)ref[i]);
     m = dlt > m ? dlt : m;
   }
-  sh[threadIdx.x] = m;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + off]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) atomicMax(d_max, (unsigned long long)__double_as_longlong(sh[0]));
+  block_max(m, d_max);
 }
 
 __global__ void k_alphas(const float* __restrict__ B, const uint8_t* __restrict__ upd, float* __restrict__ out,
@@ -1376,9 +1383,9 @@ void launch_marginals(const float* B, float* A, size_t n, hipStream_t s) {
 
 void launch_residual(const float* B, float* A, size_t n, unsigned long long* d_max, hipStream_t s) {
   if (n == 0) return;
-  unsigned g = grid_for(n, 256);
-  if (g > 4096) g = 4096;
-  hipLaunchKernelGGL(k_residual, dim3(g), dim3(256), 0, s, B, A, n, d_max);
+  // at most 8 blocks per CU; 2 float4 per thread before a small map gets fewer blocks
+  const unsigned g = std::min(grid_for(n / 4, 512), 2048u);
+  hipLaunchKernelGGL(k_residual, dim3(g), dim3(256), 0, s, (const float4*)B, (float4*)A, n / 4, d_max);
 }
 
 void launch_ref_error(const float* A, const uint8_t* upd, const float* ref, size_t n, unsigned long long* d_max,
