@@ -835,8 +835,19 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
 }
 
 // Segment sums S_q = sum of p*l over pair q's positions, in a fixed order.
-// One wavefront per tile of kTile = 512 positions; lane l owns the 8
-// consecutive positions j0 + 8l .. j0 + 8l + 7 (two 128-bit loads for FP32).
+// One wavefront per tile of kTile = 512 positions.  The kernel waits on the
+// gather of the messages (4 B each from a region written in ray order), so
+// consecutive lanes take consecutive positions: a pair's records lie close
+// together (neighbouring rays at the same step) and share the cache lines of
+// one load.  The messages then change hands through LDS: lane l sums the 8
+// consecutive positions j0 + 8l .. j0 + 8l + 7.  The indices are read once
+// per iteration and are not kept in the caches, which hold the messages.
+// Groups of kSegGroup consecutive blocks (a brick or two of pairs) run on one
+// XCD, whose L2 then serves the lines that neighbouring voxels share.
+// 13 x 640x480 at 1 cm, 30 M messages per camera: 113 us with 8 consecutive
+// positions per lane, 109 coalesced, 106 with the indices uncached, 100 with
+// the XCD groups (126-136 us without the bounds-test-free path or with groups
+// of 512 blocks).
 // Each lane sums its runs serially and writes the segments that start and
 // end inside it; the runs that cross lanes are joined by one segmented
 // inclusive scan over the 64 lanes (DPP).  Of the segments that cross tiles,
@@ -878,41 +889,37 @@ __device__ __forceinline__ int wave_scan_i(int x) {
   return x;
 }
 
-// 8 consecutive messages from p0 (a multiple of 8), zero past j1; with an
-// index array, message j is X[idx[j]]
+// Messages X[idx[j]] of positions [j0, j1) of a tile, 8 consecutive ones per
+// lane (zero past j1); sh: the wavefront's kTile floats of LDS
 template <int MT>
-__device__ __forceinline__ void load8(const typename Msg<MT>::T* __restrict__ X, const uint32_t* __restrict__ idx,
-                                      uint32_t p0, uint32_t j1, float (&x)[8]) {
-  typedef typename Msg<MT>::T T;
-  if (idx) {
-    if (p0 + 8 <= j1) {
-      const uint4 a = *reinterpret_cast<const uint4*>(idx + p0);
-      const uint4 b = *reinterpret_cast<const uint4*>(idx + p0 + 4);
-      const uint32_t ix[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+__device__ __forceinline__ void load_tile(const typename Msg<MT>::T* __restrict__ X, const uint32_t* __restrict__ idx,
+                                          uint32_t j0, uint32_t j1, uint32_t lane, float* sh, float (&x)[8]) {
+  float g[8];
+  if (j0 + kTile <= j1) {  // uniform: every tile but the last, no bounds tests
+    uint32_t ix[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = Msg<MT>::load(X, ix[i]);
-    } else {
+    for (uint32_t i = 0; i < 8; ++i) ix[i] = __builtin_nontemporal_load(idx + j0 + 64u * i + lane);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = p0 + i < j1 ? Msg<MT>::load(X, idx[p0 + i]) : 0.0f;
-    }
-    return;
-  }
-  if (p0 + 8 <= j1) {
-    constexpr int kVec = (int)(8 * sizeof(T) / sizeof(uint4));
-    union {
-      uint4 v[kVec];
-      T t[8];
-    } u;
-    const uint4* src = reinterpret_cast<const uint4*>(X + p0);
-#pragma unroll
-    for (int k = 0; k < kVec; ++k) u.v[k] = src[k];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = Msg<MT>::load(u.t, (uint32_t)i);
+    for (uint32_t i = 0; i < 8; ++i) g[i] = Msg<MT>::load(X, ix[i]);
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = p0 + i < j1 ? Msg<MT>::load(X, p0 + i) : 0.0f;
+    for (uint32_t i = 0; i < 8; ++i) {
+      const uint32_t j = j0 + 64u * i + lane;
+      g[i] = j < j1 ? Msg<MT>::load(X, idx[j]) : 0.0f;
+    }
   }
+#pragma unroll
+  for (uint32_t i = 0; i < 8; ++i) sh[64u * i + lane] = g[i];
+  // one wavefront writes and reads: LDS operations of a wavefront complete in order
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const float4 a = *reinterpret_cast<const float4*>(sh + 8u * lane);
+  const float4 b = *reinterpret_cast<const float4*>(sh + 8u * lane + 4u);
+  x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+  x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
 }
+
+constexpr uint32_t kSegGroup = 4;
 
 template <int MT>
 __global__ __launch_bounds__(256) void k_seg_sum(const uint64_t* __restrict__ heads, const uint32_t* __restrict__ tile_h0,
@@ -921,8 +928,11 @@ __global__ __launch_bounds__(256) void k_seg_sum(const uint64_t* __restrict__ he
                                                  float* __restrict__ S,
                                                  float* __restrict__ pf_v,
                                                  float* __restrict__ pl_v, float* __restrict__ mid) {
+  __shared__ __align__(16) float sh[4][kTile];
   const int lane = threadIdx.x & 63;
-  const uint32_t w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const uint32_t lb = (blockIdx.x / (8u * kSegGroup)) * (8u * kSegGroup) + (blockIdx.x & 7u) * kSegGroup +
+                      ((blockIdx.x >> 3) % kSegGroup);
+  const uint32_t w = lb * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const uint32_t j0 = w * kTile;
   if (j0 >= nlive) return;  // uniform per wavefront
   const uint32_t j1 = min(j0 + kTile, nlive);
@@ -930,7 +940,7 @@ __global__ __launch_bounds__(256) void k_seg_sum(const uint64_t* __restrict__ he
   // head bits of this lane's 8 positions (zero past nlive)
   const uint32_t hb = p0 < j1 ? (uint32_t)(heads[p0 >> 6] >> (p0 & 63)) & 0xFFu : 0u;
   float x[8];
-  load8<MT>(X, idx, p0, j1, x);
+  load_tile<MT>(X, idx, j0, j1, (uint32_t)lane, sh[threadIdx.x >> 6], x);
   const int nh = __popc(hb);
   const int incl = wave_scan_i(nh);
   const uint32_t before = tile_h0[w] + (uint32_t)(incl - nh);  // heads before p0
@@ -1307,7 +1317,8 @@ void launch_epilogue(const CamPass& a, hipStream_t s, int part) {
   const float out_scale = mo == kMsgF16 ? Msg<kMsgF16>::kOut : (mo == kMsgBF16 ? Msg<kMsgBF16>::kOut : 1.0f);
   if (a.nwin && part != 2) {
     const uint32_t ntiles = (a.nwin + kTile - 1) / kTile;
-    dim3 grid(grid_for(ntiles, 4)), block(256);
+        // whole groups of blocks for the block remapping
+    dim3 grid((grid_for(ntiles, 4) + 8 * kSegGroup - 1) / (8 * kSegGroup) * (8 * kSegGroup)), block(256);
     switch (mo) {
       case kMsgF16:
         hipLaunchKernelGGL(k_seg_sum<kMsgF16>, grid, block, 0, s, a.heads, a.tile_h0, a.nwin, (const __half*)a.Xo,
