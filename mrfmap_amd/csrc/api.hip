@@ -645,8 +645,11 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   //    d_counts / d_rayidx); then the front region (sizes d_has -> offsets
   //    d_offs) and the window region (sizes d_counts -> offsets d_has) of the
   //    final record buffer
+  // (with full-ray activation every brick on a ray's way is active; the
+  // staged ids then hold the linear brick index, below 2^23 for the sentinel)
+  const bool all_active = cam.d_walkn && c->nbricks < (1 << 23);
   launch_emit(cg, c->g, cam.d_depth, c->d_sig, c->d_bia, c->d_slot, c->d_offs, c->d_has, c->d_sell0, cam.d_front,
-              cam.d_lanes, c->d_counts, c->d_rayidx, overflow, s);
+              cam.d_lanes, c->d_counts, c->d_rayidx, overflow, all_active, s);
   if ((rc = dalloc(c, &cam.d_len_f, ntiles)) || (rc = dalloc(c, &cam.d_len_w, ntiles)) ||
       (rc = dalloc(c, &cam.d_chunk_off, (size_t)ntiles + 1)))
     return rc;
@@ -685,8 +688,9 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   // (any and wany are all zero here: cleared before the first camera, and
   // behind by the pair table of each camera)
   HIPCHK(c, hipMemsetAsync(c->d_total + 2, 0, 32, s));
-  launch_reslice(cam.d_front, cam.d_lanes, (uint32_t)npix, c->d_sell0, c->d_offs, cam.d_len_f, c->d_has, cam.d_len_w,
-                 (uint32_t)nrec_f, cam.d_inc, any, wany, (unsigned long long*)(c->d_total + 2), s);
+  launch_reslice(cam.d_front, cam.d_lanes, (uint32_t)npix, c->d_sell0, all_active ? c->d_slot : nullptr, c->d_offs,
+                 cam.d_len_f, c->d_has, cam.d_len_w, (uint32_t)nrec_f, cam.d_inc, any, wany,
+                 (unsigned long long*)(c->d_total + 2), s);
   if (c->p.brick_local_vis == MRF_VIS_BRICK_LOCAL) {
     // brick entries of the window records, while the records hold voxel ids;
     // rows past the last slice read as zero words (the window kernel's

@@ -168,8 +168,12 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 // counts[0] / counts[1] gain the row's live / live window records; per
 // wavefront counts[2] gains its rays' records (gap records included) and
 // counts[3] its rays with records.
+// SLOTS: the staged records hold (linear brick index) * 512 + voxel, and the
+// brick's slot is looked up here (neighbouring rays share their bricks).
+template <bool SLOTS>
 __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, RayRec* __restrict__ lanes,
                                                  uint32_t npix, const uint2* __restrict__ sell,
+                                                 const int32_t* __restrict__ slot,
                                                  const uint32_t* __restrict__ off_f, const uint32_t* __restrict__ len_f,
                                                  const uint32_t* __restrict__ off_w, const uint32_t* __restrict__ len_w,
                                                  uint32_t base_w, uint2* __restrict__ inc, uint8_t* __restrict__ any,
@@ -191,6 +195,16 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
   // bounds lf, lw are uniform per wavefront, so every lane takes part in the
   // shuffles)
   constexpr uint32_t kB = 8;
+  auto pool_ids = [&](uint2(&e)[kB]) {
+    if constexpr (SLOTS) {
+      int32_t sl[kB];
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u) sl[u] = slot[e[u].x != kGapVox ? e[u].x >> kBrickLog * 3 : 0u];
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u)
+        if (e[u].x != kGapVox) e[u].x = (uint32_t)sl[u] * kBrickVox + (e[u].x & (kBrickVox - 1u));
+    }
+  };
   uint64_t nl = 0, nw = 0;
   const uint32_t lf = len_f[t], lw = len_w[t];
   for (uint32_t k0 = 0; k0 < lf; k0 += kB) {
@@ -200,6 +214,7 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
       e[u] = gap;
       if (k0 + u < f.nf) e[u] = src[(size_t)(k0 + u) * kSlice];
     }
+    pool_ids(e);
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
       if (k0 + u < lf) {
@@ -219,6 +234,7 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
       e[u] = gap;
       if (k0 + u < rnw) e[u] = srcw[(size_t)(k0 + u) * kSlice];
     }
+    pool_ids(e);
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
       if (k0 + u < lw) {
@@ -1339,12 +1355,14 @@ void launch_epilogue(const CamPass& a, hipStream_t s, int part) {
                      a.npairs, a.wseg_off, a.S, a.pl_v, a.pf_v, a.mid, out_scale, a.B, a.M, a.upd, a.all_pairs);
 }
 
-void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const uint32_t* off_f,
-                    const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w, uint32_t base_w, uint2* inc,
-                    uint8_t* any, uint8_t* wany, unsigned long long* counts, hipStream_t s) {
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const int32_t* slot,
+                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
+                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, unsigned long long* counts,
+                    hipStream_t s) {
   if (npix == 0) return;
-  hipLaunchKernelGGL(k_reslice, dim3(grid_for(npix, 256)), dim3(256), 0, s, front, lanes, npix, sell, off_f, len_f,
-                     off_w, len_w, base_w, inc, any, wany, counts);
+  auto* k = slot ? k_reslice<true> : k_reslice<false>;
+  hipLaunchKernelGGL(k, dim3(grid_for(npix, 256)), dim3(256), 0, s, front, lanes, npix, sell, slot, off_f, len_f, off_w,
+                     len_w, base_w, inc, any, wany, counts);
 }
 
 void launch_brick_starts(const FrontRec* front, const RayRec* lanes, const uint32_t* len_w, uint32_t nslices,

@@ -39,11 +39,13 @@ void launch_slice_len(const uint32_t* counts, uint32_t ntiles, uint32_t* slice_l
 // lanes[t*64+l].nw window records (the ray's description, the Kahan state of
 // the front's length sum); cnt_f / cnt_w the same per tiled pixel.  A ray
 // with more records than its slice's length slice_len[t] (sized by a count
-// or a bound of it) sets *overflow.
+// or a bound of it) sets *overflow.  all_active (full-ray activation, fewer
+// than 2^23 bricks in the grid): the records hold (linear brick index) * 512
+// + voxel instead of pool ids.
 void launch_emit(const CamGeom& c, const GridGeom& g, const float* depth, const float* sig, const float* bia,
                  const int32_t* slot, const uint32_t* slice_off, const uint32_t* slice_len, uint2* sell,
                  FrontRec* front, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_w, uint32_t* overflow,
-                 hipStream_t s);
+                 bool all_active, hipStream_t s);
 
 // map evaluation of one camera's pixels (log-likelihood, expected depth,
 // accuracy and simple accuracy images in row-major pixel order, any may be
@@ -182,9 +184,11 @@ struct CamPass {
 // record (set, never cleared); counts[0] / counts[1] += the live / live
 // window records, counts[2] += all records (gap records included),
 // counts[3] += rays with records
-void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const uint32_t* off_f,
-                    const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w, uint32_t base_w, uint2* inc,
-                    uint8_t* any, uint8_t* wany, unsigned long long* counts, hipStream_t s);
+// slot (may be null): the staged records hold (linear brick index) * 512 +
+// voxel and become pool ids through it
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const int32_t* slot,
+                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
+                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, unsigned long long* counts, hipStream_t s);
 // brick entries of every window record (records still hold voxel ids):
 // bstart[(region row of the slice) + k] bit l = record k of lane l enters a
 // brick (the ray's first record, the record after a gap, or a voxel in
