@@ -1846,12 +1846,11 @@ int mrf_mlp_train(mrf_ctx* c, float* params, const float* X, const float* t, int
       const uint32_t cnt = (uint32_t)std::min<uint64_t>(batch, (uint64_t)n - off);
       launch_mlp_grad(c->d_mlp, c->d_tX, c->d_tT, c->d_tSel, (uint32_t)off, cnt, 1.0f / (float)cnt, c->d_tPart,
                       c->d_tLpart, c->stream);
-      launch_mlp_reduce(c->d_tPart, c->d_tLpart, mlp_grad_waves(cnt), c->d_tG, c->d_tLoss, 1.0 / (double)n,
-                        c->stream);
       b1t *= o->beta1;
       b2t *= o->beta2;
-      launch_adam(c->d_mlp, c->d_tG, c->d_tM, c->d_tV, lr, o->beta1, o->beta2, o->eps, (float)(1.0 - b1t),
-                  (float)(1.0 - b2t), c->stream);
+      launch_mlp_reduce_adam(c->d_tPart, c->d_tLpart, mlp_grad_waves(cnt), c->d_tLoss, 1.0 / (double)n, c->d_mlp,
+                             c->d_tM, c->d_tV, lr, o->beta1, o->beta2, o->eps, (float)(1.0 - b1t), (float)(1.0 - b2t),
+                             c->stream);
     }
     HIPCHK(c, hipGetLastError());
     double l = 0;

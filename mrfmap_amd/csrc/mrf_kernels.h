@@ -264,8 +264,10 @@ void launch_mlp_grad(const float* P, const float* X, const float* T, const uint3
                      uint32_t cnt, float scale, float* partial, double* lpart, hipStream_t s);
 void launch_mlp_reduce(const float* partial, const double* lpart, uint32_t nw, float* grad, double* loss,
                        double scale, hipStream_t s);
-void launch_adam(float* P, const float* G, float* m, float* v, float lr, float b1, float b2, float eps, float c1,
-                 float c2, hipStream_t s);
+// the same sums taken straight into Adam's step on P (moments m, v)
+void launch_mlp_reduce_adam(const float* partial, const double* lpart, uint32_t nw, double* loss, double scale,
+                            float* P, float* m, float* v, float lr, float b1, float b2, float eps, float c1, float c2,
+                            hipStream_t s);
 void launch_feat_hits(const CamGeom& c, const GridGeom& g, const float* depth, const int32_t* slot, uint32_t* hits,
                       hipStream_t s);
 void launch_feat_pairs(const uint32_t* pair_vox, const float* pair_c, const float* M, uint32_t npairs, float* pass,

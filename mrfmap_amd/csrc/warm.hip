@@ -58,15 +58,73 @@ __device__ __forceinline__ f32x4 mfma(const bf16x8& a, const bf16x8& b, const f3
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_d(float z) {
-  return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
+// gelu and its derivative from q = 2 Phi(z), the part they share
+__device__ __forceinline__ float gelu_q(float z) { return 1.0f + erff(z * 0.70710678118654752f); }
+__device__ __forceinline__ float gelu(float z, float q) { return 0.5f * z * q; }
+__device__ __forceinline__ float gelu_d(float z, float q) {
+  return fmaf(z * 0.39894228040143268f, expf(-0.5f * z * z), 0.5f * q);
 }
 
-// K slot e of layer-2 step s for lane group g -> hidden unit
-__device__ __forceinline__ int perm_k(int s, int g, int e) { return 16 * (2 * s + (e >> 2)) + 4 * g + (e & 3); }
+// a + b with b rounded first (never fused with the product that made b).  A
+// training run repeats its bits only if every step does, so which products
+// the gradient fuses into its sums is spelled out where the compiler could
+// choose, as the builds before this code chose it (gelu_d's, and of the bias
+// sums the last unit's of a tile's second half).
+__device__ __forceinline__ float add_rounded(float a, float b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
+
+// Sum over the 16 lanes of a DPP row, in every lane, in the order of xor
+// exchanges with 1, 2, 4 and 8: two quad permutations, then the mirrors of 8
+// and 16 lanes (a quad, then a half row, holds one value by then).
+template <int CTRL>
+__device__ __forceinline__ float row_add(float x) {
+  return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float row_sum(float x) { return row_add<0x140>(row_add<0x141>(row_add<0x4E>(row_add<0xB1>(x)))); }
 
 __device__ __forceinline__ float shfl_xor(float v, int m) { return __shfl_xor(v, m, 64); }
+
+// The network in LDS, one copy per block: matrices rounded to BF16 (W2 also
+// transposed, for dh1 = W2^T dz2), vectors in FP32.  Rows are padded by 16 B
+// so that the 16 rows a fragment load touches spread over the banks.  A lane's
+// fragments were some 200 separate 4 B loads from global memory, which took
+// most of a gradient step; staged, they are 40 LDS reads after 25 coalesced
+// loads per thread.
+constexpr int kPad = 8;
+struct alignas(16) NetLds {
+  unsigned short w1[kMlpHid][kMlpIn + kPad];
+  unsigned short w2[kMlpHid][kMlpHid + kPad];
+  unsigned short w2t[kMlpHid][kMlpHid + kPad];
+  float b1[kMlpHid], b2[kMlpHid], w3[kMlpHid];
+  float b3;
+};
+
+// by a block of 256 threads; every load is issued before the first is used
+template <bool W2T>
+__device__ __forceinline__ void stage_net(const float* __restrict__ P, NetLds& n) {
+  constexpr int kT = 256, k1 = kMlpHid * kMlpIn / kT, k2 = kMlpHid * kMlpHid / kT;
+  const int t = threadIdx.x;
+  float a[k1], b[k2], v = 0.f;
+  #pragma unroll
+  for (int k = 0; k < k1; ++k) a[k] = P[kMlpW1 + k * kT + t];
+  #pragma unroll
+  for (int k = 0; k < k2; ++k) b[k] = P[kMlpW2 + k * kT + t];
+  const int q = t / kMlpHid, h = t % kMlpHid;  // one vector per wave, b3 by the last
+  if (q < 3) v = P[(q == 0 ? kMlpB1 : q == 1 ? kMlpB2 : kMlpW3) + h];
+  if (t == kT - 1) v = P[kMlpB3];
+  #pragma unroll
+  for (int k = 0; k < k1; ++k) n.w1[(k * kT + t) / kMlpIn][t % kMlpIn] = bf16_bits(a[k]);
+  #pragma unroll
+  for (int k = 0; k < k2; ++k) {
+    const unsigned short u = bf16_bits(b[k]);
+    n.w2[(k * kT + t) / kMlpHid][h] = u;
+    if constexpr (W2T) n.w2t[h][(k * kT + t) / kMlpHid] = u;
+  }
+  if (q < 3) (q == 0 ? n.b1 : q == 1 ? n.b2 : n.w3)[h] = v;
+  if (t == kT - 1) n.b3 = v;
+}
 
 // Per-lane copies of the network, BF16 fragments for the MFMA operands.
 struct Frags {
@@ -76,42 +134,28 @@ struct Frags {
   float b3;
 };
 
-__device__ void load_frags(const float* __restrict__ P, int g, int c, Frags& f) {
+// elements pi(s, g, 0..7) of a 64-element row: two runs of four
+__device__ __forceinline__ bf16x8 perm_frag(const unsigned short* row, int s, int g) {
+  const uint2 lo = *reinterpret_cast<const uint2*>(row + 32 * s + 4 * g);
+  const uint2 hi = *reinterpret_cast<const uint2*>(row + 32 * s + 16 + 4 * g);
+  return __builtin_bit_cast(bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+}
+
+__device__ __forceinline__ void load_frags(const NetLds& n, int g, int c, Frags& f) {
   #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    u16x8 u;
+    f.w1[t] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&n.w1[16 * t + c][8 * g]));
     #pragma unroll
-    for (int e = 0; e < 8; ++e) u[e] = bf16_bits(P[kMlpW1 + (16 * t + c) * kMlpIn + 8 * g + e]);
-    f.w1[t] = to_bf16x8(u);
-    #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      #pragma unroll
-      for (int e = 0; e < 8; ++e) u[e] = bf16_bits(P[kMlpW2 + (16 * t + c) * kMlpHid + perm_k(s, g, e)]);
-      f.w2[t][s] = to_bf16x8(u);
-    }
+    for (int s = 0; s < 2; ++s) f.w2[t][s] = perm_frag(n.w2[16 * t + c], s, g);
     #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int h = 16 * t + 4 * g + r;
-      f.b1[4 * t + r] = P[kMlpB1 + h];
-      f.b2[4 * t + r] = P[kMlpB2 + h];
-      f.w3[4 * t + r] = P[kMlpW3 + h];
+      f.b1[4 * t + r] = n.b1[h];
+      f.b2[4 * t + r] = n.b2[h];
+      f.w3[4 * t + r] = n.w3[h];
     }
   }
-  f.b3 = P[kMlpB3];
-}
-
-// A operand of dh1 = W2^T dz2 (tile t over h1 units, step s over h2 units):
-// W2[pi(s, g, e)][16t + c]
-__device__ void load_w2t(const float* __restrict__ P, int g, int c, bf16x8 (&w2t)[4][2]) {
-  #pragma unroll
-  for (int t = 0; t < 4; ++t)
-    #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      u16x8 u;
-      #pragma unroll
-      for (int e = 0; e < 8; ++e) u[e] = bf16_bits(P[kMlpW2 + perm_k(s, g, e) * kMlpHid + 16 * t + c]);
-      w2t[t][s] = to_bf16x8(u);
-    }
+  f.b3 = n.b3;
 }
 
 // x fragment (B of layer 1) of one sample: X[i][8g .. 8g + 7], zero if !ok
@@ -133,7 +177,7 @@ __device__ __forceinline__ u16x8 load_x(const float* __restrict__ X, uint64_t i,
 // lane's hidden units; h1b: layer-2 B operand; h2: gelu(a2); returns y of the
 // lane's sample (the same value in the 4 lanes of that sample).
 struct Fwd {
-  float a1[16], a2[16], h2[16];
+  float a1[16], a2[16], h2[16], q1[16], q2[16];  // q: gelu_q of the pre-activations
   u16x8 h1u[2];  // layer-2 B operand, K slot e of step s = unit 16 (2s + e/4) + 4g + e%4
   float y;
 };
@@ -149,9 +193,11 @@ __device__ __forceinline__ void forward(const Frags& f, const u16x8& xu, Fwd& o)
     #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float a = z1[t][r] + f.b1[4 * t + r];
+      const float q = gelu_q(a);
       o.a1[4 * t + r] = a;
+      o.q1[4 * t + r] = q;
       // unit 16t + 4g + r is K slot e = 4 (t % 2) + r of step s = t / 2
-      o.h1u[t >> 1][4 * (t & 1) + r] = bf16_bits(gelu(a));
+      o.h1u[t >> 1][4 * (t & 1) + r] = bf16_bits(gelu(a, q));
     }
   const bf16x8 h0 = to_bf16x8(o.h1u[0]), h1 = to_bf16x8(o.h1u[1]);
   float part = 0.f;
@@ -162,8 +208,9 @@ __device__ __forceinline__ void forward(const Frags& f, const u16x8& xu, Fwd& o)
     #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float a = z2[r] + f.b2[4 * t + r];
-      const float h = gelu(a);
+      const float q = gelu_q(a), h = gelu(a, q);
       o.a2[4 * t + r] = a;
+      o.q2[4 * t + r] = q;
       o.h2[4 * t + r] = h;
       part += f.w3[4 * t + r] * h;
     }
@@ -179,8 +226,11 @@ __global__ void __launch_bounds__(256) k_mlp_fwd(const float* __restrict__ P, co
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
+  __shared__ NetLds net;
+  stage_net<false>(P, net);
+  __syncthreads();
   Frags f;
-  load_frags(P, g, c, f);
+  load_frags(net, g, c, f);
   const uint32_t ntiles = (n + 15) / 16;
   for (uint32_t tile = wave; tile < ntiles; tile += nwaves) {
     const uint32_t i = tile * 16 + c;
@@ -211,19 +261,23 @@ __device__ __forceinline__ bf16x8 lds_frag(const unsigned short* row, int g) {
 // Samples sel[off + i] (or off + i without sel), i < cnt, in tiles of 32;
 // loss 1/2 scale sum (y - t)^2, gradients into partial[wave][kMlpParams] and
 // lpart[wave] (the loss sum).  Every wave of the grid writes its row.
+// A step of training runs one tile per wave and fewer waves than the chip has
+// SIMDs, so the kernel is one wave's latency: 36 us at 8192 samples with the
+// network's fragments loaded one by one from global memory, the gradient
+// accumulators spilled (616 B per lane) and the 16-lane sums through LDS;
+// 24 us staged, without spills and with the sums in DPP.
 __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ P, const float* __restrict__ X,
                                                   const float* __restrict__ T, const uint32_t* __restrict__ sel,
                                                   uint32_t off, uint32_t cnt, float scale,
                                                   float* __restrict__ partial, double* __restrict__ lpart) {
   __shared__ WaveLds lds_all[kGradWaves];
+  __shared__ NetLds net;
+  stage_net<true>(P, net);
+  __syncthreads();
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int wib = threadIdx.x >> 6;
   WaveLds& L = lds_all[wib];
   const uint32_t wave = blockIdx.x * kGradWaves + wib;
-  Frags f;
-  load_frags(P, g, c, f);
-  bf16x8 w2t[4][2];
-  load_w2t(P, g, c, w2t);
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 gw2[4][4], gw1[4][2];
   #pragma unroll
@@ -242,8 +296,13 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ P, c
   for (uint32_t base = blockIdx.x * kGradWaves; base < ntiles; base += gridDim.x * kGradWaves) {
     const uint32_t tile = base + wib;
     const bool tile_ok = tile < ntiles;
-    #pragma unroll
+    #pragma unroll 1
     for (int hf = 0; hf < 2; ++hf) {
+      // the network's fragments are read from LDS for each half, not kept
+      // across the loop: with the gradient accumulators they would spill
+      asm volatile("" ::: "memory");
+      Frags f;
+      load_frags(net, g, c, f);
       const uint32_t li = tile * kTileS + hf * 16 + c;
       const bool ok = tile_ok && li < cnt;
       const uint64_t i = ok ? (sel ? (uint64_t)sel[off + li] : (uint64_t)off + li) : 0;
@@ -263,24 +322,24 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ P, c
         for (int r = 0; r < 4; ++r) {
           const int k = 4 * t + r;
           gw3[k] += dy * o.h2[k];
-          const float dz = f.w3[k] * dy * gelu_d(o.a2[k]);
-          gb2[k] += dz;
+          const float dz = f.w3[k] * dy * gelu_d(o.a2[k], o.q2[k]);
+          gb2[k] = add_rounded(gb2[k], dz);
           const unsigned short b = bf16_bits(dz);
           du[t >> 1][4 * (t & 1) + r] = b;
           L.dz2[16 * t + 4 * g + r][hf * 16 + c] = b;
           L.h1[16 * t + 4 * g + r][hf * 16 + c] = o.h1u[t >> 1][4 * (t & 1) + r];
         }
       const bf16x8 db0 = to_bf16x8(du[0]), db1 = to_bf16x8(du[1]);
-      // dh1 = W2^T dz2, dz1 = dh1 gelu'(a1)
+      // dh1 = W2^T dz2 (A: W2[pi(s, g, e)][16t + c]), dz1 = dh1 gelu'(a1)
       #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        f32x4 dh = mfma(w2t[t][0], db0, zero);
-        dh = mfma(w2t[t][1], db1, dh);
+        f32x4 dh = mfma(perm_frag(net.w2t[16 * t + c], 0, g), db0, zero);
+        dh = mfma(perm_frag(net.w2t[16 * t + c], 1, g), db1, dh);
         #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int k = 4 * t + r;
-          const float dz = dh[r] * gelu_d(o.a1[k]);
-          gb1[k] += dz;
+          const float gd = gelu_d(o.a1[k], o.q1[k]), dz = dh[r] * gd;
+          gb1[k] = hf == 1 && k == 15 ? fmaf(dh[r], gd, gb1[k]) : add_rounded(gb1[k], dz);
           L.dz1[16 * t + 4 * g + r][hf * 16 + c] = bf16_bits(dz);
         }
       }
@@ -302,13 +361,11 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ P, c
   }
   // reduce the per-sample sums over the 16 lanes of a group
   #pragma unroll
-  for (int k = 0; k < 16; ++k)
-    #pragma unroll
-    for (int m = 1; m < 16; m <<= 1) {
-      gb1[k] += shfl_xor(gb1[k], m);
-      gb2[k] += shfl_xor(gb2[k], m);
-      gw3[k] += shfl_xor(gw3[k], m);
-    }
+  for (int k = 0; k < 16; ++k) {
+    gb1[k] = row_sum(gb1[k]);
+    gb2[k] = row_sum(gb2[k]);
+    gw3[k] = row_sum(gw3[k]);
+  }
   #pragma unroll
   for (int m = 1; m < 64; m <<= 1) {
     gb3 += shfl_xor(gb3, m);
@@ -341,32 +398,66 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ P, c
   }
 }
 
-// grad[j] = sum over waves in order; loss[0] += sum of the wave losses x scale
-__global__ void k_mlp_reduce(const float* __restrict__ partial, const double* __restrict__ lpart, uint32_t nw,
-                             float* __restrict__ grad, double* __restrict__ loss, double scale) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < kMlpParams) {
-    float s = 0.f;
-    for (uint32_t w = 0; w < nw; ++w) s += partial[(size_t)w * kMlpParams + j];
-    grad[j] = s;
-  }
-  if (j == 0 && loss) {
-    double s = 0.0;
-    for (uint32_t w = 0; w < nw; ++w) s += lpart[w];
-    loss[0] += s * scale;
-  }
-}
+// Adam's moments and step (c1, c2: the bias corrections)
+struct Adam {
+  float *P, *m, *v;
+  float lr, b1, b2, eps, c1, c2;
+};
 
-__global__ void k_adam(float* __restrict__ P, const float* __restrict__ G, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= kMlpParams) return;
-  const float g = G[j];
-  const float mj = b1 * m[j] + (1.f - b1) * g;
-  const float vj = b2 * v[j] + (1.f - b2) * g * g;
-  m[j] = mj;
-  v[j] = vj;
-  P[j] -= lr * (mj / c1) / (sqrtf(vj / c2) + eps);
+// grad[j] = sum of partial over the nw waves in order, or, with ADAM, that sum
+// taken straight into the parameters' step; loss[0] += sum of the wave losses
+// x scale.  A block owns 64 parameters: its waves bring the rows of a chunk
+// into LDS together (the chunk's loads are all in flight), one wave adds them
+// in order (the order of the sums is part of the result: training repeats it
+// step by step).  At 8192 samples (256 rows) 5.3 us with Adam, against 65 us
+// for one thread per parameter over all rows in 25 blocks, and 5 us for Adam
+// as a launch of its own.
+constexpr int kRedCols = 64, kRedWaves = 16, kRedRows = 256;
+template <bool ADAM>
+__global__ __launch_bounds__(kRedCols* kRedWaves) void k_mlp_reduce(const float* __restrict__ partial,
+                                                                    const double* __restrict__ lpart, uint32_t nw,
+                                                                    float* __restrict__ grad,
+                                                                    double* __restrict__ loss, double scale, Adam a) {
+  __shared__ float sh[kRedRows][kRedCols];
+  __shared__ double lsh[kRedRows];
+  const uint32_t col = threadIdx.x & (kRedCols - 1), wv = threadIdx.x / kRedCols;
+  const uint32_t j = blockIdx.x * kRedCols + col;
+  const bool in = j < (uint32_t)kMlpParams, losses = blockIdx.x == 0 && loss;
+  float s = 0.f;
+  double l = 0.0;
+  for (uint32_t w0 = 0; w0 < nw; w0 += kRedRows) {
+    const uint32_t n = min((uint32_t)kRedRows, nw - w0);
+    float v[kRedRows / kRedWaves];
+    #pragma unroll
+    for (int k = 0; k < kRedRows / kRedWaves; ++k) {
+      const uint32_t w = k * kRedWaves + wv;
+      v[k] = in && w < n ? partial[(size_t)(w0 + w) * kMlpParams + j] : 0.f;
+    }
+    #pragma unroll
+    for (int k = 0; k < kRedRows / kRedWaves; ++k) sh[k * kRedWaves + wv][col] = v[k];
+    if (losses && threadIdx.x < n) lsh[threadIdx.x] = lpart[w0 + threadIdx.x];
+    __syncthreads();
+    if (wv == 0) {
+      #pragma unroll 16
+      for (uint32_t w = 0; w < n; ++w) s += sh[w][col];
+    } else if (losses && threadIdx.x == kRedCols) {
+      #pragma unroll 8
+      for (uint32_t w = 0; w < n; ++w) l += lsh[w];
+    }
+    __syncthreads();
+  }
+  if (wv == 0 && in) {
+    if constexpr (ADAM) {
+      const float mj = a.b1 * a.m[j] + (1.f - a.b1) * s;
+      const float vj = a.b2 * a.v[j] + (1.f - a.b2) * s * s;
+      a.m[j] = mj;
+      a.v[j] = vj;
+      a.P[j] -= a.lr * (mj / a.c1) / (sqrtf(vj / a.c2) + a.eps);
+    } else {
+      grad[j] = s;
+    }
+  }
+  if (losses && threadIdx.x == kRedCols) loss[0] += l * scale;
 }
 
 // ---------------------------------------------------------------- features
@@ -511,13 +602,15 @@ void launch_mlp_grad(const float* P, const float* X, const float* T, const uint3
 
 void launch_mlp_reduce(const float* partial, const double* lpart, uint32_t nw, float* grad, double* loss,
                        double scale, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(kMlpParams, 256)), dim3(256), 0, s, partial, lpart, nw, grad, loss,
-                     scale);
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3(blocks(kMlpParams, kRedCols)), dim3(kRedCols * kRedWaves), 0, s,
+                     partial, lpart, nw, grad, loss, scale, Adam{});
 }
 
-void launch_adam(float* P, const float* G, float* m, float* v, float lr, float b1, float b2, float eps, float c1,
-                 float c2, hipStream_t s) {
-  hipLaunchKernelGGL(k_adam, dim3(blocks(kMlpParams, 256)), dim3(256), 0, s, P, G, m, v, lr, b1, b2, eps, c1, c2);
+void launch_mlp_reduce_adam(const float* partial, const double* lpart, uint32_t nw, double* loss, double scale,
+                            float* P, float* m, float* v, float lr, float b1, float b2, float eps, float c1, float c2,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(k_mlp_reduce<true>, dim3(blocks(kMlpParams, kRedCols)), dim3(kRedCols * kRedWaves), 0, s,
+                     partial, lpart, nw, nullptr, loss, scale, Adam{P, m, v, lr, b1, b2, eps, c1, c2});
 }
 
 void launch_feat_pairs(const uint32_t* pair_vox, const float* pair_c, const float* M, uint32_t npairs, float* pass,
