@@ -85,6 +85,7 @@ struct mrf_ctx {
   mrf_params p;
   std::vector<float> sig_tab, bia_tab;
   bool user_tables = false;
+  bool const_model = false;  // every cell's sigma and bias are constants
   int tab_rows = 0, tab_cols = 0;
   float *d_sig = nullptr, *d_bia = nullptr;
   GridGeom g;
@@ -372,6 +373,13 @@ CamGeom make_geom(const mrf_ctx* c, const Camera& cam) {
   return g;
 }
 
+// Whether every cell of a sensor-model table is a constant
+bool constant_cells(const std::vector<float>& tab, int lookup_n) {
+  for (size_t i = 0; i < tab.size(); ++i)
+    if (i % (size_t)lookup_n != 0 && tab[i] != 0.0f) return false;
+  return true;
+}
+
 // (Re)build the sensor-model tables so that every camera's lookup cells exist.
 int ensure_tables(mrf_ctx* c, int rows, int cols) {
   const int ln = c->p.lookup_n;
@@ -391,6 +399,7 @@ int ensure_tables(mrf_ctx* c, int rows, int cols) {
       c->sig_tab[i * ln + j] = c->p.const_sigmasq_poly[j];
       c->bia_tab[i * ln + j] = c->p.const_bias_poly[j];
     }
+  c->const_model = constant_cells(c->sig_tab, ln) && constant_cells(c->bia_tab, ln);
   dfree(&c->d_sig);
   dfree(&c->d_bia);
   ++c->epoch;  // a captured iteration holds the old table pointers
@@ -993,6 +1002,7 @@ CamPass cam_pass(mrf_ctx* c, size_t ci) {
   a.sig = c->d_sig;
   a.bia = c->d_bia;
   a.lookup_n = c->p.lookup_n;
+  a.const_model = c->const_model;
   a.msg_type = c->p.msg_dtype;
   a.ray_sched = c->ray_sched < 0 ? kSchedF8W4 : c->ray_sched;
   a.brick_local = c->p.brick_local_vis == MRF_VIS_BRICK_LOCAL;
@@ -1394,6 +1404,7 @@ int mrf_create(const mrf_params* p, mrf_ctx** out) {
     c->sig_tab.assign(p->depth_sigma_lookup, p->depth_sigma_lookup + cells * p->lookup_n);
     c->bia_tab.assign(p->depth_bias_lookup, p->depth_bias_lookup + cells * p->lookup_n);
     c->user_tables = true;
+    c->const_model = constant_cells(c->sig_tab, p->lookup_n) && constant_cells(c->bia_tab, p->lookup_n);
     c->tab_rows = p->rows;
     c->tab_cols = p->cols;
     if ((rc = dalloc(c, &c->d_sig, c->sig_tab.size())) || (rc = dalloc(c, &c->d_bia, c->bia_tab.size()))) {

@@ -86,15 +86,6 @@ __device__ __forceinline__ float lane63(float x) {
 constexpr float kNegHalfLog2e = -0.72134752044448170f;
 __device__ __forceinline__ float gauss_a(float u) { return 0.398942f * __builtin_amdgcn_exp2f((u * u) * kNegHalfLog2e); }
 
-// psi(s; d) = N(d; s + bias(s), (3 sigma(s))^2) (depth_potential,
-// gvdbkernels.cu:57-72), with the likelihood width 3 sigma(s) evaluated
-// from sigma's coefficients times 3 (sig3)
-__device__ __forceinline__ float depth_psi(float s, float d, const Poly& sig3, const Poly& bia) {
-  const float diff = fabsf(d - (s + bia(s)));
-  const float inv = __builtin_amdgcn_rcpf(sig3(s));
-  return gauss_a(diff * inv) * inv;
-}
-
 // ---------------------------------------------------------------- segments
 // A camera's incidences are stored pair-major: pair q owns positions
 // [pair_off[q], pair_off[q+1]).  Segment heads are marked in a bitmask and
@@ -623,7 +614,21 @@ __device__ __forceinline__ void win_issue(Rsrc rx, const uint2 (&e)[UW], float (
 struct WinRay {
   float z0, inv, d;
   Poly sig3, bia;  // 3 sigma(z) (the likelihood width) and bias(z)
+  float rsig3;     // 1 / sig3.c0
 };
+
+// a = 0.398942 e^{-u^2/2} and psi(s; d) = N(d; s + bias(s), (3 sigma(s))^2) =
+// a / (3 sigma(s)) (depth_potential, gvdbkernels.cu:57-72).  CS: every lookup
+// cell's sigma and bias are constants (c1 = c2 = 0), so the polynomials and
+// the reciprocal leave the loop with the same bits: fmaf(z, fmaf(z, 0, 0), c0)
+// is c0.
+template <bool CS>
+__device__ __forceinline__ void win_psi(const WinRay& r, float s, float& ap, float& ps) {
+  const float diff = fabsf(r.d - (s + (CS ? r.bia.c0 : r.bia(s))));
+  const float inv = CS ? r.rsig3 : __builtin_amdgcn_rcpf(r.sig3(s));
+  ap = gauss_a(diff * inv);
+  ps = ap * inv;
+}
 
 // depth at the exit of a record: z0 + (travelled chord length) * inv
 __device__ __forceinline__ float win_depth(const WinRay& r, const Kahan& kS, float ln) {
@@ -631,25 +636,27 @@ __device__ __forceinline__ float win_depth(const WinRay& r, const Kahan& kS, flo
 }
 
 // terms of one record shared by both passes: a = l log2 n, vpsi, n
+template <bool CS>
 __device__ __forceinline__ void win_terms(const WinRay& r, const Kahan& kL, const Kahan& kS, float ln, float lnn,
                                           float& a, float& vpsi, float& nn) {
   a = ln * lnn;
   const float s = win_depth(r, kS, ln);
-  const float ps = depth_psi(s, r.d, r.sig3, r.bia);
+  float ap, ps;
+  win_psi<CS>(r, s, ap, ps);
   // a gap or padding record (log2 n = 0) gets a vpsi but n = 1 exactly, so
   // its tau vpsi (1 - n) is exactly 0; its own message is never read
   vpsi = __builtin_amdgcn_exp2f(kL.at(a)) * ps;
   nn = __builtin_amdgcn_exp2f(lnn);
 }
 
-template <int UW>
+template <int UW, bool CS>
 __device__ __forceinline__ void win_pass1(const WinRay& r, uint32_t k0, uint32_t nw, const float (&ln)[UW],
                                           const float (&x)[UW], Kahan& kL, Kahan& kS, float& T) {
 #pragma unroll
   for (int u = 0; u < UW; ++u) {
     const bool valid = k0 + u < nw;
     float a, vpsi, nn;
-    win_terms(r, kL, kS, ln[u], x[u], a, vpsi, nn);
+    win_terms<CS>(r, kL, kS, ln[u], x[u], a, vpsi, nn);
     T += valid ? vpsi * (1.0f - nn) : 0.0f;
     kL.add(a);  // a = 0 and l = 0 past the lane's last record: no select needed
     kS.add(ln[u]);
@@ -664,49 +671,57 @@ __device__ __forceinline__ void win_pass1(const WinRay& r, uint32_t k0, uint32_t
 // the row's word in bsw; the restore at gvdbkernels.cu:708-715 tests the
 // accumulated tau), and only such taus enter T.  The terms are those of
 // win_terms, so a ray whose restarts change nothing gets the T of pass 1.
+// The per-lane conditions are kept as wavefront masks in scalar registers (nz:
+// the lanes that have a counted tau; bsw: the rows' brick-entry words, a
+// batch loaded together), so a record costs two selects for the restart and
+// one for the tau and the batch has no branches: with a branch and a scalar
+// load per record the compiler waited for each word in turn.  4 x 160x120 at
+// 4 cm (one wave per SIMD, bound by latency): 48.3 -> 42.8 us per camera pass
+// together with the constant sensor model; 13 x 640x480 at 1 cm (bound by
+// memory traffic): 190 us either way.
 constexpr float kFtzMin = 0x1p-126f;
 
-template <int UW>
+template <int UW, bool CS>
 __device__ __forceinline__ void win_pass1_bl(const WinRay& r, uint32_t k0, uint32_t nw, const float (&ln)[UW],
-                                             const float (&x)[UW], const uint64_t* __restrict__ bsw, uint32_t l,
-                                             Kahan& kL, Kahan& kS, float& T, bool& nz) {
+                                             const float (&x)[UW], const uint64_t* __restrict__ bsw, Kahan& kL,
+                                             Kahan& kS, float& T, uint64_t& nz) {
+  uint64_t w[UW];
+#pragma unroll
+  for (int u = 0; u < UW; ++u) w[u] = bsw[k0 + u];
 #pragma unroll
   for (int u = 0; u < UW; ++u) {
-    const bool valid = k0 + u < nw;
-    const bool restart = valid && !nz && ((bsw[k0 + u] >> l) & 1ull) != 0ull;
+    const uint64_t valid = __ballot(k0 + u < nw);
+    const bool restart = __builtin_amdgcn_inverse_ballot_w64(w[u] & valid & ~nz);
     kL.s = restart ? 0.0f : kL.s;
     kL.c = restart ? 0.0f : kL.c;
     const float lnn = x[u];
     const float a = ln[u] * lnn;
     const float s = win_depth(r, kS, ln[u]);
-    const float diff = fabsf(r.d - (s + r.bia(s)));
-    const float inv = __builtin_amdgcn_rcpf(r.sig3(s));
-    const float uu = diff * inv;
-    const float ap = gauss_a(uu);
-    const float ps = ap * inv;  // depth_psi's product order
+    float ap, ps;
+    win_psi<CS>(r, s, ap, ps);
     const float V = __builtin_amdgcn_exp2f(kL.at(a));
     const float nn = __builtin_amdgcn_exp2f(lnn);
     const float b = V * (1.0f - nn);
     // every factor at least 2^-126 (log2 n = 0, a gap or padding record, gives b = 0)
-    const bool counted = valid && fminf(fminf(ap, ps), fminf(b, b * ps)) >= kFtzMin;
-    T += counted ? (V * ps) * (1.0f - nn) : 0.0f;
-    nz = nz || counted;
+    const uint64_t counted = valid & __ballot(fminf(fminf(ap, ps), fminf(b, b * ps)) >= kFtzMin);
+    T += __builtin_amdgcn_inverse_ballot_w64(counted) ? (V * ps) * (1.0f - nn) : 0.0f;
+    nz |= counted;
     kL.add(a);  // a = 0 and l = 0 past the lane's last record: no select needed
     kS.add(ln[u]);
   }
 }
 
-template <int UW, bool BL>
+template <int UW, bool BL, bool CS>
 __device__ __forceinline__ void win_pass1_any(const WinRay& r, uint32_t k0, uint32_t nw, const float (&ln)[UW],
-                                              const float (&x)[UW], const uint64_t* __restrict__ bsw, uint32_t l,
-                                              Kahan& kL, Kahan& kS, float& T, bool& nz) {
+                                              const float (&x)[UW], const uint64_t* __restrict__ bsw, Kahan& kL,
+                                              Kahan& kS, float& T, uint64_t& nz) {
   if constexpr (BL)
-    win_pass1_bl<UW>(r, k0, nw, ln, x, bsw, l, kL, kS, T, nz);
+    win_pass1_bl<UW, CS>(r, k0, nw, ln, x, bsw, kL, kS, T, nz);
   else
-    win_pass1<UW>(r, k0, nw, ln, x, kL, kS, T);
+    win_pass1<UW, CS>(r, k0, nw, ln, x, kL, kS, T);
 }
 
-template <int MO, int UW>
+template <int MO, int UW, bool CS>
 __device__ __forceinline__ void win_pass2(const WinRay& r, uint32_t k0, uint32_t nw, const float (&ln)[UW],
                                           const float (&x)[UW], float T, Rsrc ro, uint32_t lane_off, Kahan& kL,
                                           Kahan& kS, float& P) {
@@ -715,7 +730,7 @@ __device__ __forceinline__ void win_pass2(const WinRay& r, uint32_t k0, uint32_t
   for (int u = 0; u < UW; ++u) {
     const bool valid = k0 + u < nw;
     float a, vpsi, nn;
-    win_terms(r, kL, kS, ln[u], x[u], a, vpsi, nn);
+    win_terms<CS>(r, kL, kS, ln[u], x[u], a, vpsi, nn);
     const float tau = vpsi * (1.0f - nn);
     const float R = (T - P) - tau;
     const float mu1 = P + vpsi;
@@ -729,7 +744,7 @@ __device__ __forceinline__ void win_pass2(const WinRay& r, uint32_t k0, uint32_t
   }
 }
 
-template <int MI, int MO, int UW, bool BL>
+template <int MI, int MO, int UW, bool BL, bool CS>
 __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ lanes, const uint32_t* __restrict__ len_w,
                                                     uint32_t nslices, const uint32_t* __restrict__ chunk_off,
                                                     const float* __restrict__ partial, const uint2* __restrict__ inc,
@@ -773,6 +788,7 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
   r.sig3.c0 *= 3.0f;
   r.sig3.c1 *= 3.0f;
   r.sig3.c2 *= 3.0f;
+  r.rsig3 = __builtin_amdgcn_rcpf(r.sig3.c0);
   r.z0 = rec.z0;
   r.inv = rec.inv_norm;
   r.d = rec.depth;
@@ -789,7 +805,7 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
   uint2 e[UW];
   // pass 1
   float T = 0.0f;  // sum of the taus: positive terms, a plain sum
-  bool nz = false;
+  uint64_t nz = 0;
   const uint64_t* bsw = nullptr;
   if constexpr (BL) {
     // the pre pass enters the window with the visibility sum of the front
@@ -822,11 +838,11 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
   for (uint32_t k0 = 0;; k0 += 2 * UW) {  // bounded by the slice's longest ray: uniform control flow
     win_issue<MI, UW>(rx, e, lB, xB);
     win_load<UW>(rr, lr, k0 + 2 * UW, e);
-    win_pass1_any<UW, BL>(r, k0, nw, lA, xA, bsw, l, kL, kS, T, nz);
+    win_pass1_any<UW, BL, CS>(r, k0, nw, lA, xA, bsw, kL, kS, T, nz);
     if (k0 + UW >= lws) break;
     win_issue<MI, UW>(rx, e, lA, xA);
     win_load<UW>(rr, lr, k0 + 3 * UW, e);
-    win_pass1_any<UW, BL>(r, k0 + UW, nw, lB, xB, bsw, l, kL, kS, T, nz);
+    win_pass1_any<UW, BL, CS>(r, k0 + UW, nw, lB, xB, bsw, kL, kS, T, nz);
     if (k0 + 2 * UW >= lws) break;
   }
   if (rec.cell_flags & kInfTerm) T += __builtin_amdgcn_exp2f(kL.at(0.0f));  // decided at traversal
@@ -841,11 +857,11 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
   for (uint32_t k0 = 0;; k0 += 2 * UW) {
     win_issue<MI, UW>(rx, e, lB, xB);
     win_load<UW>(rr, lr, k0 + 2 * UW, e);
-    win_pass2<MO, UW>(r, k0, nw, lA, xA, T, ro, lo, kL, kS, P);
+    win_pass2<MO, UW, CS>(r, k0, nw, lA, xA, T, ro, lo, kL, kS, P);
     if (k0 + UW >= lws) break;
     win_issue<MI, UW>(rx, e, lA, xA);
     win_load<UW>(rr, lr, k0 + 3 * UW, e);
-    win_pass2<MO, UW>(r, k0 + UW, nw, lB, xB, T, ro, lo, kL, kS, P);
+    win_pass2<MO, UW, CS>(r, k0 + UW, nw, lB, xB, T, ro, lo, kL, kS, P);
     if (k0 + 2 * UW >= lws) break;
   }
 }
@@ -1293,14 +1309,10 @@ void launch_ray_t(const CamPass& a, hipStream_t s, int part) {
   if (part == 1) return;
   const uint32_t blocks = (a.nslices * kSlice + 63) / 64;
   const unsigned nb = (blocks + 7) / 8 * 8;  // multiple of the 8 XCDs for the block remapping
-  if (a.brick_local)
-    hipLaunchKernelGGL((k_ray_window<MI, MO, UW, true>), dim3(nb), dim3(64), 0, s, a.lanes, a.len_w, a.nslices,
-                       a.chunk_off, a.partial, a.inc, a.base_w, Xi, a.npairs, (typename Msg<MO>::T*)a.Xo, a.sig, a.bia,
-                       a.lookup_n, a.front, a.bstart, a.tail);
-  else
-    hipLaunchKernelGGL((k_ray_window<MI, MO, UW, false>), dim3(nb), dim3(64), 0, s, a.lanes, a.len_w, a.nslices,
-                       a.chunk_off, a.partial, a.inc, a.base_w, Xi, a.npairs, (typename Msg<MO>::T*)a.Xo, a.sig, a.bia,
-                       a.lookup_n, a.front, a.bstart, a.tail);
+  auto* k = a.brick_local ? (a.const_model ? k_ray_window<MI, MO, UW, true, true> : k_ray_window<MI, MO, UW, true, false>)
+                          : (a.const_model ? k_ray_window<MI, MO, UW, false, true> : k_ray_window<MI, MO, UW, false, false>);
+  hipLaunchKernelGGL(k, dim3(nb), dim3(64), 0, s, a.lanes, a.len_w, a.nslices, a.chunk_off, a.partial, a.inc, a.base_w,
+                     Xi, a.npairs, (typename Msg<MO>::T*)a.Xo, a.sig, a.bia, a.lookup_n, a.front, a.bstart, a.tail);
 }
 
 template <int MI, int MO>

@@ -169,6 +169,7 @@ struct CamPass {
   const float* sig;        // sensor-model lookup tables
   const float* bia;
   int lookup_n;
+  bool const_model;        // every cell's sigma and bias are constants
   int msg_type;
   int ray_sched;           // RaySched
   // pre-pass visibility restarted at brick entries until a tau survives
