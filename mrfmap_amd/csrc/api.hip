@@ -141,7 +141,7 @@ struct mrf_ctx {
 
   std::vector<Camera> cams;
   bool geom_dirty = true;
-  int ray_sched = -1;      // chosen RaySched, -1 until autotuned
+  int ray_sched = kSchedF16W8;  // RaySched in use (choose_schedule)
   // captured BP iteration: valid while no buffer it uses is reallocated
   uint64_t epoch = 0;      // bumped whenever geometry or pool buffers change
   hipGraphExec_t gexec = nullptr;
@@ -149,7 +149,6 @@ struct mrf_ctx {
   int launch_mode = MRF_LAUNCH_GRAPH;
   bool graph_ok = true;    // false once a capture failed
   bool sched_forced = false;
-  double autotune_ms = 0.0;
   // learned warm start: per-voxel feature accumulators, feature rows,
   // predictions, the fallback snapshot, MLP parameters and training scratch
   float *d_wpass = nullptr, *d_wmsum = nullptr, *d_wmmax = nullptr, *d_wdelta = nullptr;
@@ -790,6 +789,20 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
 
 CamPass cam_pass(mrf_ctx* c, size_t ci);
 
+// Ray-kernel schedule (records loaded ahead in the front and the window
+// kernel) by size.  16 x 8 is the best or within 1 % of it from 20 k rays at
+// 4 cm to 300 k at 1 cm with up to 17 M pairs per camera (window kernel 60.9
+// us against 69.6 with 4 ahead and 62.6 with 16 for 320x240 at 2 cm, 191
+// against 207 and 195 for 640x480 at 1 cm).  With 58 M pairs per camera
+// (10x10x3 m at 1 cm) the messages no longer fit the last-level cache and the
+// longer gathers want 16 ahead: 210 against 224 us.  The line is at 32 M
+// pairs, 128 MB of messages, half of that cache.
+int choose_schedule(const mrf_ctx* c) {
+  uint32_t np = 0;
+  for (const Camera& cam : c->cams) np = std::max(np, cam.npairs);
+  return np > (32u << 20) ? kSchedF16W16 : kSchedF16W8;
+}
+
 int prepare(mrf_ctx* c) {
   if (!c->geom_dirty) return MRF_OK;
   ++c->epoch;  // camera lists and per-pass scratch are rebuilt below
@@ -924,6 +937,7 @@ int prepare(mrf_ctx* c) {
     }
     c->Xo_bytes = xout;
   }
+  if (!c->sched_forced) c->ray_sched = choose_schedule(c);
   c->geom_dirty = false;
   return MRF_OK;
 }
@@ -1004,52 +1018,11 @@ CamPass cam_pass(mrf_ctx* c, size_t ci) {
   a.lookup_n = c->p.lookup_n;
   a.const_model = c->const_model;
   a.msg_type = c->p.msg_dtype;
-  a.ray_sched = c->ray_sched < 0 ? kSchedF8W4 : c->ray_sched;
+  a.ray_sched = c->ray_sched;
   a.brick_local = c->p.brick_local_vis == MRF_VIS_BRICK_LOCAL;
   a.bstart = cam.d_bstart;
   a.tail = cam.d_tail;
   return a;
-}
-
-// Pick the ray-kernel schedule (lanes per ray x loads in flight) by timing
-// each candidate twice on the camera with the most incidences.  Only the
-// pass's message scratch is touched, not beliefs.
-int autotune(mrf_ctx* c) {
-  if (c->cams.empty()) return MRF_OK;
-  auto t0 = std::chrono::steady_clock::now();
-  size_t best_cam = 0;
-  for (size_t i = 1; i < c->cams.size(); ++i)
-    if (c->cams[i].nupd > c->cams[best_cam].nupd) best_cam = i;
-  hipEvent_t e0, e1;
-  HIPCHK(c, hipEventCreate(&e0));
-  HIPCHK(c, hipEventCreate(&e1));
-  float best = 1e30f;
-  int pick = kSchedF8W4;
-  for (int sched = 0; sched < kNumSched; ++sched) {
-    CamPass a = cam_pass(c, best_cam);
-    a.ray_sched = sched;
-    float tmin = 1e30f;
-    for (int rep = 0; rep < 2; ++rep) {
-      launch_pair_msgs(a, c->stream);
-      HIPCHK(c, hipEventRecord(e0, c->stream));
-      launch_ray_messages(a, c->stream);
-      HIPCHK(c, hipEventRecord(e1, c->stream));
-      HIPCHK(c, hipEventSynchronize(e1));
-      float ms = 0;
-      HIPCHK(c, hipEventElapsedTime(&ms, e0, e1));
-      tmin = std::min(tmin, ms);
-    }
-    if (tmin < best) {
-      best = tmin;
-      pick = sched;
-    }
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  HIPCHK(c, hipGetLastError());
-  c->ray_sched = pick;
-  c->autotune_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  return MRF_OK;
 }
 
 // Evaluate the current map from camera geometry cg (depth already on the
@@ -1393,7 +1366,7 @@ int mrf_create(const mrf_params* p, mrf_ctx** out) {
     return rc;
   }
   {
-    const uint32_t flags[2] = {1u, 2u};  // defined before the autotuner's first pair pass
+    const uint32_t flags[2] = {1u, 2u};  // defined from the start; every call sets them
     if (hipMemcpy(c->d_all_pairs, flags, sizeof(flags), hipMemcpyHostToDevice) != hipSuccess) {
       mrf_destroy(c);
       return MRF_E_HIP;
@@ -1531,7 +1504,6 @@ static int run_inference(mrf_ctx* c, const uint32_t* ids, int n_ids, int max_ite
   if (rc) return rc;
   auto t1 = std::chrono::steady_clock::now();
   if (dirty) s.t_geometry_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
-  if (c->ray_sched < 0 && (rc = autotune(c))) return rc;
   const size_t nvox = c->slot_lin.size() * (size_t)kBrickVox;
   // reset M_c of the selected cameras (GVDBInference.cpp:128-134); the
   // first iteration refreshes every pair's message
@@ -1671,7 +1643,7 @@ static int run_inference(mrf_ctx* c, const uint32_t* ids, int n_ids, int max_ite
   s.t_iters_ms = titer;
   s.t_total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   s.ray_sched = c->ray_sched;
-  s.t_autotune_ms = c->autotune_ms;
+  s.t_autotune_ms = 0.0;  // the schedule follows from the sizes
   s.warm = warm_state;
   s.ref_error = rerr;
   if (st) *st = s;

@@ -15,8 +15,8 @@ inline int msg_out_type(int t) {
 inline size_t msg_bytes(int type) { return type == kMsgF32 ? 4 : 2; }
 
 // Schedules of the ray-message kernel: records loaded ahead of their
-// arithmetic in the front loop (F) and in the window passes (W).  Picked per
-// workload by the autotuner in api.hip.
+// arithmetic in the front loop (F) and in the window passes (W).  Picked by
+// size in api.hip (choose_schedule); MRF_RAY_SCHED forces one.
 enum RaySched { kSchedF8W4 = 0, kSchedF8W8 = 1, kSchedF16W4 = 2, kSchedF16W8 = 3, kSchedF4W4 = 4, kSchedF16W16 = 5,
                 kNumSched = 6 };
 
