@@ -39,7 +39,7 @@ inline void check(int rc, mrf_ctx* c, const char* where) {
   }
 }
 
-/* Gives the large device blocks that destroyed contexts left with the
+/* Gives the device blocks that destroyed contexts left with the
  * library back to the HIP runtime (mrf_release_device_cache). */
 inline void release_device_cache() { check(mrf_release_device_cache(), nullptr, "mrf_release_device_cache"); }
 

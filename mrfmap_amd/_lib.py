@@ -151,7 +151,7 @@ def load():
 
 
 def release_device_cache():
-    """Give the large device blocks the library keeps after freeing them back
+    """Give the device blocks the library keeps after freeing them back
     to the HIP runtime (mrf_release_device_cache)."""
     check(load().mrf_release_device_cache())
 

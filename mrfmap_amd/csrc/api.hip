@@ -226,23 +226,33 @@ int fail(mrf_ctx* c, int code, const std::string& msg) {
       return fail(ctx, MRF_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));             \
   } while (0)
 
-// Process-wide cache of large device blocks.  A context's lists take tens
-// of GB (85 GB for 64 keyframes); when they are freed and a new context
-// allocates as much again, the runtime takes seconds to provide the memory
-// (a 64-keyframe build: 0.86 s in a fresh process, 4.3-4.5 s after a
-// context of that size was closed, whose frees took 2.4 s).  Blocks of at
-// least kCacheMin bytes are therefore kept on free (after the device has
-// finished with them) and handed out again for requests of up to their size
-// and at least 4/5 of it.  The cache keeps at most 3/4 of the device's
-// memory, gives everything back when an allocation fails, and is emptied by
+// Process-wide cache of device blocks.  A context makes some 25 allocations
+// per camera and as many frees when it is closed or a camera is traversed
+// again; hipMalloc takes 25-40 us and hipFree 80-180 us (4 x 160x120: 15 of
+// the 18 ms of a map built from nothing; 13 x 640x480: 44 of 140 ms), and for
+// lists of tens of GB the runtime takes seconds to provide the memory again
+// (a 64-keyframe build: 0.86 s in a fresh process, 4.3-4.5 s after a context
+// of that size was closed, whose frees took 2.4 s).  Blocks are therefore
+// kept on free (after the device has finished with them) and handed out again
+// for requests of up to their size and at least 4/5 of it.  Sizes below 32 MiB
+// are rounded up to eighths of a power of two, so that slightly different
+// requests share blocks; larger blocks keep their size, since lists may take
+// most of the device.  The cache keeps at most 3/4 of the device's memory, gives
+// everything back when an allocation fails, and is emptied by
 // mrf_release_device_cache(); MRF_NO_DEVICE_CACHE=1 switches it off.
 struct BlockCache {
   std::mutex mu;
-  std::unordered_map<void*, std::pair<size_t, int>> live;  // large blocks in use: bytes, device
+  std::unordered_map<void*, std::pair<size_t, int>> live;  // blocks in use: bytes, device
   std::multimap<std::pair<int, size_t>, void*> idle;        // (device, bytes) -> kept block
   size_t kept = 0;
 };
-constexpr size_t kCacheMin = size_t(32) << 20;
+
+size_t block_size(size_t bytes) {
+  if (bytes >= size_t(32) << 20) return bytes;
+  size_t step = 512;  // 4 KiB and below: multiples of 512 B
+  while (step * 16 <= bytes) step *= 2;
+  return (bytes + step - 1) / step * step;
+}
 
 BlockCache& block_cache() {
   static BlockCache* bc = new BlockCache;  // never destroyed: frees may run during static destruction
@@ -272,7 +282,8 @@ void release_idle(BlockCache& bc, int dev) {
 
 hipError_t dev_malloc(void** p, size_t bytes) {
   *p = nullptr;
-  if (bytes < kCacheMin || !cache_enabled()) return hipMalloc(p, bytes);
+  if (!cache_enabled()) return hipMalloc(p, bytes);
+  bytes = block_size(bytes);
   int dev = 0;
   (void)hipGetDevice(&dev);
   BlockCache& bc = block_cache();

@@ -49,7 +49,7 @@ class GVDBInference:
         self._cam_shapes = {}
 
     def close(self):
-        """Destroy the context.  Its large device blocks stay with the library
+        """Destroy the context.  Its device blocks stay with the library
         for the next context; ``mrfmap_amd.release_device_cache()`` gives them
         back to the HIP runtime."""
         if getattr(self, "_h", None):
