@@ -43,6 +43,7 @@ struct Camera {
   RayRec* d_lanes = nullptr;       // one per lane of every slice (tiled pixel order)
   uint32_t* d_len_f = nullptr;     // front records per lane of each slice
   uint32_t* d_len_w = nullptr;     // window records per lane of each slice
+  bool listed = false;             // the lists below are those of the current pose and active bricks
   uint32_t nslices = 0;
   uint32_t nrays = 0;              // rays with at least one record
   uint2* d_inc = nullptr;          // sliced records {pair | gap, length}: front region, then window region
@@ -95,6 +96,7 @@ struct mrf_ctx {
 
   std::vector<int32_t> h_slot;   // brick directory: linear brick index -> slot or -1
   std::vector<int32_t> slot_lin; // slot -> linear brick index
+  size_t listed_slots = 0;       // slots when the cameras were last listed
   int32_t* d_slot = nullptr;
   uint8_t* d_bflags = nullptr;
   size_t cap_slots = 0;
@@ -635,6 +637,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
     launch_scatter_pairs(cam.d_pair_vox, cam.d_M, cam.npairs, c->d_A, c->stream);
   }
   free_camera_lists(cam);
+  cam.listed = false;
   const CamGeom cg = make_geom(c, cam);
   const size_t npix = (size_t)num_tiled_pixels(cg);
   const uint32_t ntiles = (uint32_t)(npix / kSlice);
@@ -795,6 +798,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   HIPCHK(c, hipStreamSynchronize(s));
   HIPCHK(c, hipGetLastError());
   dfree(&cam.d_walkn);  // after the sync: a free waits for the device
+  cam.listed = true;
   return MRF_OK;
 }
 
@@ -818,9 +822,16 @@ int prepare(mrf_ctx* c) {
   if (!c->geom_dirty) return MRF_OK;
   ++c->epoch;  // camera lists and per-pass scratch are rebuilt below
   int rc;
-  // 1. activation
+  // A keyframe's lists follow from its pose, depth and sensor model and from
+  // the active bricks on its rays.  With full-ray activation these are the
+  // bricks its own rays mark, which stay active, so only new and moved
+  // keyframes are walked and listed again (six 640x480 keyframes at 1 cm, one
+  // moved: 5 ms per camera not traversed); with endpoint activation a new
+  // brick may lie on any ray, so new bricks list every keyframe again.
+  // 1. activation by the keyframes to list
   HIPCHK(c, hipMemsetAsync(c->d_bflags, 0, (size_t)c->nbricks, c->stream));
   for (Camera& cam : c->cams) {
+    if (cam.listed) continue;
     const CamGeom cg = make_geom(c, cam);
     if (c->p.activation == MRF_ACT_FULL_RAY) {
       const size_t npix = (size_t)num_tiled_pixels(cg);
@@ -841,19 +852,22 @@ int prepare(mrf_ctx* c) {
       c->slot_lin.push_back(lin);
     }
   }
+  if (c->p.activation == MRF_ACT_ENDPOINT && c->slot_lin.size() != c->listed_slots)
+    for (Camera& cam : c->cams) cam.listed = false;
+  c->listed_slots = c->slot_lin.size();
   if ((rc = ensure_pool(c, c->slot_lin.size()))) return rc;
   // the directory is uploaded by every build, grown or not: the device copy
   // is not initialised when the context is created (4 B per brick of the grid)
   HIPCHK(c, hipMemcpyAsync(c->d_slot, c->h_slot.data(), c->h_slot.size() * 4, hipMemcpyHostToDevice, c->stream));
-  // 3. traversal lists and pairs of every camera; the voxel flags of the
-  //    pair numbering start cleared (each camera clears its own behind)
+  // 3. traversal lists and pairs of the cameras to list; the voxel flags of
+  //    the pair numbering start cleared (each camera clears its own behind)
   {
     const size_t nvox = c->slot_lin.size() * (size_t)kBrickVox;
     if ((rc = ensure_vflags(c, std::max<size_t>(nvox, 1)))) return rc;
     launch_zero_words(c->d_vflag, (2 * nvox + 3) / 4 * 4, c->stream);  // the byte flags any, wany
   }
   for (Camera& cam : c->cams)
-    if ((rc = traverse_camera(c, cam))) return rc;
+    if (!cam.listed && (rc = traverse_camera(c, cam))) return rc;
   // 3b. voxels where some camera has window records; per camera, its
   //     front-only pairs there (their log2 n keeps changing after the first
   //     iterations of a call, the others' stops)
@@ -1476,6 +1490,7 @@ int mrf_set_pose(mrf_ctx* c, uint32_t id, const float pose[16], int layout) {
   } else {
     std::memcpy(cam.pose, pose, sizeof(cam.pose));
   }
+  cam.listed = false;
   c->geom_dirty = true;
   return MRF_OK;
 }
