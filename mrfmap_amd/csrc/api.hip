@@ -818,12 +818,12 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
 CamPass cam_pass(mrf_ctx* c, size_t ci);
 
 // Ray-kernel schedule (records loaded ahead in the front and the window
-// kernel) by size.  16 x 8 is the best or within 2 % of it from 20 k rays at
-// 4 cm to 300 k at 1 cm with up to 17 M pairs per camera (window kernel 58.0
-// us against 65.1 with 4 ahead and 60.6 with 16 for 320x240 at 2 cm, 174
-// against 181 and 188 for 640x480 at 1 cm).  With 58 M pairs per camera
+// kernel) by size.  16 x 8 is the best or within 1 % of it from 20 k rays at
+// 4 cm to 300 k at 1 cm with up to 17 M pairs per camera (window kernel 60.9
+// us against 69.6 with 4 ahead and 62.6 with 16 for 320x240 at 2 cm, 191
+// against 207 and 195 for 640x480 at 1 cm).  With 58 M pairs per camera
 // (10x10x3 m at 1 cm) the messages no longer fit the last-level cache and the
-// longer gathers want 16 ahead: 192 against 199 us.  The line is at 32 M
+// longer gathers want 16 ahead: 210 against 224 us.  The line is at 32 M
 // pairs, 128 MB of messages, half of that cache.
 int choose_schedule(const mrf_ctx* c) {
   uint32_t np = 0;
