@@ -40,15 +40,13 @@ struct Camera {
   int rows = 0, cols = 0;
   float* d_depth = nullptr;
   FrontRec* d_front = nullptr;     // one per lane of every slice (tiled pixel order)
-  SkirtRec* d_skirt = nullptr;     // the same
   RayRec* d_lanes = nullptr;       // one per lane of every slice (tiled pixel order)
   uint32_t* d_len_f = nullptr;     // front records per lane of each slice
-  uint32_t* d_len_s = nullptr;     // skirt records per lane of each slice
   uint32_t* d_len_w = nullptr;     // window records per lane of each slice
   bool listed = false;             // the lists below are those of the current pose and active bricks
   uint32_t nslices = 0;
   uint32_t nrays = 0;              // rays with at least one record
-  uint2* d_inc = nullptr;          // sliced records {pair | gap, length}: front, skirt and window regions
+  uint2* d_inc = nullptr;          // sliced records {pair | gap, length}: front region, then window region
   uint32_t* d_walkn = nullptr;     // full-ray activation: bound of the records per tiled pixel
   uint8_t* d_lnn = nullptr;        // per pair: voxel -> ray message log2 n (input-side message type)
   uint2* d_dyn = nullptr;          // front-only pairs at voxels where some camera has window records: {pair, voxel}
@@ -62,7 +60,7 @@ struct Camera {
   uint2* d_dcr = nullptr;             // per changing chunk: {first row, rows} in d_dfront
   uint2* d_fspan = nullptr;           // per lane of every slice: first front record, front records to sum
   uint64_t nstatic = 0;            // live records in such chunks
-  uint64_t nrec = 0, base_s = 0, base_w = 0;  // padded records; first records of the skirt and window regions
+  uint64_t nrec = 0, base_w = 0;   // padded records; first record of the window region
   uint64_t nupd = 0;               // live incidences
   uint64_t nwin = 0;               // live window incidences (window positions)
   uint64_t nlist = 0;              // records without the slice padding
@@ -78,8 +76,8 @@ struct Camera {
   uint32_t* d_chunk_off = nullptr; // nslices + 1: first front chunk of each slice
   uint4* d_chunk_desc = nullptr;
   uint32_t nchunks = 0;
-  uint64_t* d_bstart = nullptr;    // MRF_VIS_BRICK_LOCAL: brick-entry word per skirt and window row of every slice
-  uint8_t* d_tail = nullptr;       // MRF_VIS_BRICK_LOCAL: per lane, front records in the brick that follows them
+  uint64_t* d_bstart = nullptr;    // MRF_VIS_BRICK_LOCAL: brick-entry word per window row of every slice
+  uint8_t* d_tail = nullptr;       // MRF_VIS_BRICK_LOCAL: per lane, front records in the first window brick
 };
 
 }  // namespace
@@ -135,7 +133,6 @@ struct mrf_ctx {
 
   // scratch
   uint32_t *d_counts = nullptr, *d_has = nullptr, *d_offs = nullptr, *d_rayidx = nullptr;
-  uint32_t *d_scnt = nullptr, *d_soff = nullptr;  // skirt counts; skirt offsets, then sizes, per slice
   size_t cap_pix = 0;
   uint64_t* d_scan_tmp = nullptr;
   size_t cap_scan = 0;
@@ -431,12 +428,9 @@ int ensure_pixel_scratch(mrf_ctx* c, size_t npix) {
   dfree(&c->d_has);
   dfree(&c->d_offs);
   dfree(&c->d_rayidx);
-  dfree(&c->d_scnt);
-  dfree(&c->d_soff);
   int rc;
   if ((rc = dalloc(c, &c->d_counts, npix)) || (rc = dalloc(c, &c->d_has, npix)) ||
-      (rc = dalloc(c, &c->d_offs, npix)) || (rc = dalloc(c, &c->d_rayidx, npix)) ||
-      (rc = dalloc(c, &c->d_scnt, npix)) || (rc = dalloc(c, &c->d_soff, npix)))
+      (rc = dalloc(c, &c->d_offs, npix)) || (rc = dalloc(c, &c->d_rayidx, npix)))
     return rc;
   c->cap_pix = npix;
   return MRF_OK;
@@ -599,10 +593,8 @@ void free_camera_lists(Camera& cam) {
   dfree(&cam.d_dyn);
   cam.ndyn = 0;
   dfree(&cam.d_front);
-  dfree(&cam.d_skirt);
   dfree(&cam.d_lanes);
   dfree(&cam.d_len_f);
-  dfree(&cam.d_len_s);
   dfree(&cam.d_len_w);
   dfree(&cam.d_inc);
   dfree(&cam.d_win_idx);
@@ -620,7 +612,7 @@ void free_camera_lists(Camera& cam) {
   cam.nchunks = 0;
   cam.nrays = 0;
   cam.nslices = 0;
-  cam.nrec = cam.base_s = cam.base_w = cam.nupd = cam.nwin = cam.nlist = 0;
+  cam.nrec = cam.base_w = cam.nupd = cam.nwin = cam.nlist = 0;
   cam.npairs = cam.nwp = 0;
 }
 
@@ -667,46 +659,41 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   HIPCHK(c, hipGetLastError());
   if (nrec0 >= 0x7FFFFFF0ull) return fail(c, MRF_E_LIMIT, "more than 2^31 incidence records in one camera");
   if ((rc = ensure_sell0(c, std::max<uint64_t>(nrec0, 1))) || (rc = dalloc(c, &cam.d_front, npix)) ||
-      (rc = dalloc(c, &cam.d_skirt, npix)) || (rc = dalloc(c, &cam.d_lanes, npix)))
+      (rc = dalloc(c, &cam.d_lanes, npix)))
     return rc;
   uint32_t* overflow = reinterpret_cast<uint32_t*>(c->d_total + 6);
   launch_zero_words(overflow, 8, s);
-  // 2. the emission splits each ray into front, skirt and window (counts into
-  //    d_counts / d_scnt / d_rayidx); then the front region (sizes d_has ->
-  //    offsets d_offs), the skirt region (sizes d_soff + ntiles -> offsets
-  //    d_soff) and the window region (sizes d_counts -> offsets d_has) of the
+  // 2. the emission splits each ray into front and window (counts into
+  //    d_counts / d_rayidx); then the front region (sizes d_has -> offsets
+  //    d_offs) and the window region (sizes d_counts -> offsets d_has) of the
   //    final record buffer
   // (with full-ray activation every brick on a ray's way is active; the
   // staged ids then hold the linear brick index, below 2^23 for the sentinel)
   const bool all_active = cam.d_walkn && c->nbricks < (1 << 23);
   launch_emit(cg, c->g, cam.d_depth, c->d_sig, c->d_bia, c->d_slot, c->d_offs, c->d_has, c->d_sell0, cam.d_front,
-              cam.d_skirt, cam.d_lanes, c->d_counts, c->d_scnt, c->d_rayidx,
-              c->p.brick_local_vis == MRF_VIS_BRICK_LOCAL ? kFrontU : kSkirtU, overflow, all_active, s);
-  if ((rc = dalloc(c, &cam.d_len_f, ntiles)) || (rc = dalloc(c, &cam.d_len_s, ntiles)) || (rc = dalloc(c, &cam.d_len_w, ntiles)) ||
+              cam.d_lanes, c->d_counts, c->d_rayidx, overflow, all_active, s);
+  if ((rc = dalloc(c, &cam.d_len_f, ntiles)) || (rc = dalloc(c, &cam.d_len_w, ntiles)) ||
       (rc = dalloc(c, &cam.d_chunk_off, (size_t)ntiles + 1)))
     return rc;
   // ... and the front chunks, ceil(len_f / kChunk) per slice that has window
-  // records (sizes d_counts -> chunk_off); the four totals in one readback
-  uint64_t* tot = c->d_total + 2;
+  // records (sizes d_counts -> chunk_off); the three totals in one readback
+  uint64_t* tot3 = c->d_total + 2;
   launch_slice_len(c->d_counts, ntiles, cam.d_len_f, c->d_has, s);
-  launch_exclusive_scan(c->d_has, c->d_offs, ntiles, c->d_scan_tmp, tot, s);
-  launch_slice_len(c->d_scnt, ntiles, cam.d_len_s, c->d_soff + ntiles, s);  // npix = 64 ntiles words
-  launch_exclusive_scan(c->d_soff + ntiles, c->d_soff, ntiles, c->d_scan_tmp, tot + 3, s);
+  launch_exclusive_scan(c->d_has, c->d_offs, ntiles, c->d_scan_tmp, tot3, s);
   launch_slice_len(c->d_rayidx, ntiles, cam.d_len_w, c->d_counts, s);
-  launch_exclusive_scan(c->d_counts, c->d_has, ntiles, c->d_scan_tmp, tot + 1, s);
+  launch_exclusive_scan(c->d_counts, c->d_has, ntiles, c->d_scan_tmp, tot3 + 1, s);
   launch_chunk_counts(cam.d_len_f, cam.d_len_w, ntiles, c->d_counts, s);
-  launch_exclusive_scan(c->d_counts, cam.d_chunk_off, (size_t)ntiles + 1, c->d_scan_tmp, tot + 2, s);
-  uint64_t t4[4] = {0, 0, 0, 0};
-  HIPCHK(c, hipMemcpyAsync(t4, tot, sizeof(t4), hipMemcpyDeviceToHost, s));
+  launch_exclusive_scan(c->d_counts, cam.d_chunk_off, (size_t)ntiles + 1, c->d_scan_tmp, tot3 + 2, s);
+  uint64_t t3[3] = {0, 0, 0};
+  HIPCHK(c, hipMemcpyAsync(t3, tot3, sizeof(t3), hipMemcpyDeviceToHost, s));
   HIPCHK(c, hipStreamSynchronize(s));
-  const uint64_t nrec_f = t4[0], nrec_w = t4[1], base_w = nrec_f + t4[3];
-  cam.nchunks = (uint32_t)t4[2];
-  const uint64_t nrec = base_w + nrec_w;
+  const uint64_t nrec_f = t3[0], nrec_w = t3[1];
+  cam.nchunks = (uint32_t)t3[2];
+  const uint64_t nrec = nrec_f + nrec_w;
   HIPCHK(c, hipGetLastError());
   if (nrec >= 0x7FFFFFF0ull) return fail(c, MRF_E_LIMIT, "more than 2^31 incidence records in one camera");
   cam.nrec = nrec;
-  cam.base_s = nrec_f;
-  cam.base_w = base_w;
+  cam.base_w = nrec_f;
   cam.nslices = ntiles;
   if ((rc = dalloc(c, &cam.d_inc, nrec))) return rc;
   // 3. the records into their regions; the voxels of live records (any) and
@@ -723,18 +710,18 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   // (any and wany are all zero here: cleared before the first camera, and
   // behind by the pair table of each camera)
   HIPCHK(c, hipMemsetAsync(c->d_total + 2, 0, 32, s));
-  launch_reslice(cam.d_front, cam.d_skirt, cam.d_lanes, (uint32_t)npix, c->d_sell0, all_active ? c->d_slot : nullptr,
-                 c->d_offs, cam.d_len_f, c->d_soff, cam.d_len_s, (uint32_t)nrec_f, c->d_has, cam.d_len_w,
-                 (uint32_t)base_w, cam.d_inc, any, wany, (unsigned long long*)(c->d_total + 2), s);
+  launch_reslice(cam.d_front, cam.d_lanes, (uint32_t)npix, c->d_sell0, all_active ? c->d_slot : nullptr, c->d_offs,
+                 cam.d_len_f, c->d_has, cam.d_len_w, (uint32_t)nrec_f, cam.d_inc, any, wany,
+                 (unsigned long long*)(c->d_total + 2), s);
   if (c->p.brick_local_vis == MRF_VIS_BRICK_LOCAL) {
-    // brick entries of the skirt and window records, while the records hold
-    // voxel ids; rows past the last slice read as zero words (the window
-    // kernel's batches may look up to 31 rows past a slice's longest ray)
-    const size_t wrows = (size_t)((nrec - nrec_f) / kSlice);
+    // brick entries of the window records, while the records hold voxel ids;
+    // rows past the last slice read as zero words (the window kernel's
+    // batches may look up to 16 rows past a slice's longest ray)
+    const size_t wrows = (size_t)(nrec_w / kSlice);
     if ((rc = dalloc(c, &cam.d_bstart, wrows + 32)) || (rc = dalloc(c, &cam.d_tail, npix))) return rc;
     launch_zero_words(cam.d_bstart + wrows, 32 * sizeof(uint64_t), s);
-    launch_brick_starts(cam.d_front, cam.d_skirt, cam.d_lanes, cam.d_len_s, cam.d_len_w, ntiles, cam.d_inc,
-                        (uint32_t)nrec_f, cam.d_bstart, cam.d_tail, s);
+    launch_brick_starts(cam.d_front, cam.d_lanes, cam.d_len_w, ntiles, cam.d_inc, (uint32_t)nrec_f, cam.d_bstart,
+                        cam.d_tail, s);
   }
   // one allocation for the partial sums, the static sums and the masks of
   // changing records (per chunk and lane each)
@@ -786,7 +773,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   uint32_t* acc_w = c->d_acc;
   uint32_t* acc_f = c->d_acc + 2 * (size_t)np;
   uint32_t* acc_r = c->d_acc + 4 * (size_t)np;
-  launch_pair_lengths(cam.d_inc, nrec, base_w, pid, acc_f, acc_r, np, c->d_keys_in, c->d_vals_in, nwp, s);
+  launch_pair_lengths(cam.d_inc, nrec, nrec_f, pid, acc_f, acc_r, np, c->d_keys_in, c->d_vals_in, nwp, s);
   // 6. window segments: the window records stably sorted by pair
   HIPCHK(c, sort_window((uint32_t)nrec_w, wbits, c->d_keys_in, c->d_keys_out, c->d_vals_in, cam.d_win_idx,
                         c->d_sort_tmp, c->sort_tmp_bytes, s));
@@ -798,7 +785,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   }
   launch_window_offsets(c->d_keys_out, whead, (uint32_t)nwin, nwp, cam.d_wseg_off, s);
   // C with its window part summed per segment, and the front messages
-  launch_pair_finish(cam.d_inc + base_w, c->d_keys_out, cam.d_win_idx, (uint32_t)nwin, nwp, acc_w, acc_f, acc_r, np,
+  launch_pair_finish(cam.d_inc + nrec_f, c->d_keys_out, cam.d_win_idx, (uint32_t)nwin, nwp, acc_w, acc_f, acc_r, np,
                      cam.d_pair_c, cam.d_pair_sf, s);
   // 7. window segment head bitmask and per-tile head counts
   const size_t nwords_w = nwin / 64 + 1, ntiles_w = nwin / kTile + 1;
@@ -1014,9 +1001,6 @@ CamPass cam_pass(mrf_ctx* c, size_t ci) {
   a.lanes = cam.d_lanes;
   a.len_f = cam.d_len_f;
   a.len_w = cam.d_len_w;
-  a.skirt = cam.d_skirt;
-  a.len_s = cam.d_len_s;
-  a.base_s = (uint32_t)cam.base_s;
   a.nslices = cam.nslices;
   a.inc = cam.d_inc;
   a.win_idx = cam.d_win_idx;
@@ -1461,7 +1445,6 @@ void mrf_destroy(mrf_ctx* c) {
   dfree(&c->d_tSel); dfree(&c->d_tLpart); dfree(&c->d_tLoss);
   drop_graph(c);
   dfree(&c->d_counts); dfree(&c->d_has); dfree(&c->d_offs); dfree(&c->d_rayidx);
-  dfree(&c->d_scnt); dfree(&c->d_soff);
   dfree(&c->d_scan_tmp); dfree(&c->d_total);
   dev_free(c->d_fscan_tmp); dfree(&c->d_all_pairs);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1968,11 +1951,9 @@ int mrf_get_traversal(mrf_ctx* c, uint32_t id, int64_t* n_rays, int64_t* n_recor
   // compact the sliced lists back to per-ray lists in tile order
   const size_t npix = (size_t)cam.nslices * kSlice;
   std::vector<FrontRec> front(npix);
-  std::vector<SkirtRec> skirt(npix);
   std::vector<RayRec> lanes(npix);
   std::vector<uint2> sell(cam.nrec);
   HIPCHK(c, hipMemcpy(front.data(), cam.d_front, npix * sizeof(FrontRec), hipMemcpyDeviceToHost));
-  HIPCHK(c, hipMemcpy(skirt.data(), cam.d_skirt, npix * sizeof(SkirtRec), hipMemcpyDeviceToHost));
   HIPCHK(c, hipMemcpy(lanes.data(), cam.d_lanes, npix * sizeof(RayRec), hipMemcpyDeviceToHost));
   if (cam.nrec) {
     uint2* tmp = nullptr;
@@ -1986,9 +1967,8 @@ int mrf_get_traversal(mrf_ctx* c, uint32_t id, int64_t* n_rays, int64_t* n_recor
   uint64_t off = 0, r = 0;
   for (size_t pix = 0; pix < npix; ++pix) {
     const FrontRec& F = front[pix];
-    const SkirtRec& S = skirt[pix];
     const RayRec& L = lanes[pix];
-    const uint32_t n = F.nf + S.n + L.nw;
+    const uint32_t n = F.nf + L.nw;
     if (n == 0) continue;
     if (rays) {
       uint32_t* o = rays + 6 * r;
@@ -2001,9 +1981,7 @@ int mrf_get_traversal(mrf_ctx* c, uint32_t id, int64_t* n_rays, int64_t* n_recor
     }
     if (records)
       for (uint32_t k = 0; k < n; ++k) {
-        const uint2 e = k < F.nf         ? sell[F.off + (size_t)k * kSlice]
-                        : k < F.nf + S.n ? sell[S.off + (size_t)(k - F.nf) * kSlice]
-                                         : sell[L.off_w + (size_t)(k - F.nf - S.n) * kSlice];
+        const uint2 e = k < F.nf ? sell[F.off + (size_t)k * kSlice] : sell[L.off_w + (size_t)(k - F.nf) * kSlice];
         records[2 * (off + k)] = e.x;
         records[2 * (off + k) + 1] = e.y;
       }

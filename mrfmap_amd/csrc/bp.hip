@@ -149,9 +149,9 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 }
 
 // ---------------------------------------------------------------- list layout
-// Copy every ray's records into the front, skirt and window regions of the
-// final record buffer (sliced: lane l of slice t at region offset + k * 64 +
-// l), padding each lane to its slice's length with gap records.  One wavefront
+// Copy every ray's records into the front and window regions of the final
+// record buffer (sliced: lane l of slice t at region offset + k * 64 + l),
+// padding each lane to its slice's length with gap records.  One wavefront
 // is one slice, so record k of the 64 rays moves together: per row the
 // voxel flags any[v] = 1 (every live record) and wany[v] = 1 (live window
 // records) are set, skipping a lane whose voxel equals that of the ray to
@@ -162,71 +162,88 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 // SLOTS: the staged records hold (linear brick index) * 512 + voxel, and the
 // brick's slot is looked up here (neighbouring rays share their bricks).
 template <bool SLOTS>
-__global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, SkirtRec* __restrict__ skirt,
-                                                 RayRec* __restrict__ lanes, uint32_t npix,
-                                                 const uint2* __restrict__ sell, const int32_t* __restrict__ slot,
+__global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, RayRec* __restrict__ lanes,
+                                                 uint32_t npix, const uint2* __restrict__ sell,
+                                                 const int32_t* __restrict__ slot,
                                                  const uint32_t* __restrict__ off_f, const uint32_t* __restrict__ len_f,
-                                                 const uint32_t* __restrict__ off_s, const uint32_t* __restrict__ len_s,
-                                                 uint32_t base_s, const uint32_t* __restrict__ off_w,
-                                                 const uint32_t* __restrict__ len_w, uint32_t base_w,
-                                                 uint2* __restrict__ inc, uint8_t* __restrict__ any,
+                                                 const uint32_t* __restrict__ off_w, const uint32_t* __restrict__ len_w,
+                                                 uint32_t base_w, uint2* __restrict__ inc, uint8_t* __restrict__ any,
                                                  uint8_t* __restrict__ wany, unsigned long long* __restrict__ counts) {
   const uint32_t ray = blockIdx.x * blockDim.x + threadIdx.x;
   if (ray >= npix) return;  // uniform per wavefront: npix is a multiple of 64
   const uint32_t t = ray >> 6, l = ray & 63u;
   const FrontRec f = front[ray];
-  const uint32_t rns = skirt[ray].n, rnw = lanes[ray].nw;
+  const uint32_t rnw = lanes[ray].nw;
   const uint2* __restrict__ src = sell + f.off;
-  const uint32_t fo = off_f[t] + l, so = base_s + off_s[t] + l, wo = base_w + off_w[t] + l;
+  const uint32_t fo = off_f[t] + l, wo = base_w + off_w[t] + l;
   const uint2 gap = make_uint2(kGapVox, 0u);
   // a voxel this lane need not flag: the left or the upper ray has it too
   auto dup = [&](uint32_t v) {
     const uint32_t left = (uint32_t)__shfl_up((int)v, 1, 64), up = (uint32_t)__shfl_up((int)v, 8, 64);
     return ((l & 7u) != 0u && left == v) || (l >= 8u && up == v);
   };
+  // rows in batches of kB: the batch's loads are in flight together (the
+  // bounds lf, lw are uniform per wavefront, so every lane takes part in the
+  // shuffles)
+  constexpr uint32_t kB = 8;
+  auto pool_ids = [&](uint2(&e)[kB]) {
+    if constexpr (SLOTS) {
+      int32_t sl[kB];
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u) sl[u] = slot[e[u].x != kGapVox ? e[u].x >> kBrickLog * 3 : 0u];
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u)
+        if (e[u].x != kGapVox) e[u].x = (uint32_t)sl[u] * kBrickVox + (e[u].x & (kBrickVox - 1u));
+    }
+  };
   uint64_t nl = 0, nw = 0;
-  // n records of the lane from src to inc + to, len rows of the slice, in
-  // batches of kB: the batch's loads are in flight together (len is uniform
-  // per wavefront, so every lane takes part in the shuffles)
-  auto copy = [&](const uint2* from, uint32_t n, size_t to, uint32_t len, bool window) {
-    constexpr uint32_t kB = 8;
-    for (uint32_t k0 = 0; k0 < len; k0 += kB) {
-      uint2 e[kB];
+  const uint32_t lf = len_f[t], lw = len_w[t];
+  for (uint32_t k0 = 0; k0 < lf; k0 += kB) {
+    uint2 e[kB];
 #pragma unroll
-      for (uint32_t u = 0; u < kB; ++u) {
-        e[u] = gap;
-        if (k0 + u < n) e[u] = from[(size_t)(k0 + u) * kSlice];
+    for (uint32_t u = 0; u < kB; ++u) {
+      e[u] = gap;
+      if (k0 + u < f.nf) e[u] = src[(size_t)(k0 + u) * kSlice];
+    }
+    pool_ids(e);
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      if (k0 + u < lf) {
+        inc[fo + (size_t)(k0 + u) * kSlice] = e[u];
+        const bool live = e[u].x != kGapVox;
+        nl += (uint64_t)__popcll(__ballot(live));
+        const bool d = dup(e[u].x);
+        if (live && !d) any[e[u].x] = 1;
       }
-      if constexpr (SLOTS) {
-        int32_t sl[kB];
+    }
+  }
+  const uint2* __restrict__ srcw = src + (size_t)f.nf * kSlice;
+  for (uint32_t k0 = 0; k0 < lw; k0 += kB) {
+    uint2 e[kB];
 #pragma unroll
-        for (uint32_t u = 0; u < kB; ++u) sl[u] = slot[e[u].x != kGapVox ? e[u].x >> kBrickLog * 3 : 0u];
+    for (uint32_t u = 0; u < kB; ++u) {
+      e[u] = gap;
+      if (k0 + u < rnw) e[u] = srcw[(size_t)(k0 + u) * kSlice];
+    }
+    pool_ids(e);
 #pragma unroll
-        for (uint32_t u = 0; u < kB; ++u)
-          if (e[u].x != kGapVox) e[u].x = (uint32_t)sl[u] * kBrickVox + (e[u].x & (kBrickVox - 1u));
-      }
-#pragma unroll
-      for (uint32_t u = 0; u < kB; ++u) {
-        if (k0 + u < len) {
-          inc[to + (size_t)(k0 + u) * kSlice] = e[u];
-          const bool live = e[u].x != kGapVox;
-          const uint64_t c = (uint64_t)__popcll(__ballot(live));
-          nl += c;
-          if (window) nw += c;
-          const bool d = dup(e[u].x);
-          if (live && !d) {
-            any[e[u].x] = 1;
-            if (window) wany[e[u].x] = 1;
-          }
+    for (uint32_t u = 0; u < kB; ++u) {
+      if (k0 + u < lw) {
+        inc[wo + (size_t)(k0 + u) * kSlice] = e[u];
+        const bool live = e[u].x != kGapVox;
+        const uint64_t n = (uint64_t)__popcll(__ballot(live));
+        nl += n;
+        nw += n;
+        const bool d = dup(e[u].x);
+        if (live && !d) {
+          any[e[u].x] = 1;
+          wany[e[u].x] = 1;
         }
       }
     }
-  };
-  copy(src, f.nf, fo, len_f[t], false);
-  copy(src + (size_t)f.nf * kSlice, rns, so, len_s[t], false);
-  copy(src + (size_t)(f.nf + rns) * kSlice, rnw, wo, len_w[t], true);
+  }
   // the ray's records (gap records included) and whether it has any
-  uint32_t nr = f.nf + rns + rnw;
+  uint32_t nr = f.nf + rnw;
   const uint64_t nray = (uint64_t)__popcll(__ballot(nr != 0u));
   for (int o = 32; o > 0; o >>= 1) nr += (uint32_t)__shfl_xor((int)nr, o, 64);
   if (l == 0) {
@@ -236,49 +253,42 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, S
     if (nray) atomicAdd(&counts[3], (unsigned long long)nray);
   }
   front[ray].off = fo;
-  skirt[ray].off = so;
   lanes[ray].off_w = wo;
 }
 
-// Brick entries of the skirt and window records, one wavefront per slice,
-// while the records still hold voxel ids (slot * 512 + voxel in the brick): a
-// record enters a brick when it is a voxel record and the previous record of
-// its ray is a gap record, lies in another slot, or does not exist.  The 64
-// lanes' flags of a row form one 64-bit word.  tail[lane]: when the first
-// record past the front continues the brick of the last front record, the
+// Brick entries of the window records, one wavefront per slice, while the
+// records still hold voxel ids (slot * 512 + voxel in the brick): record k
+// of lane l enters a brick when it is a voxel record and the previous record
+// of its ray is a gap record, lies in another slot, or does not exist.  The
+// 64 lanes' flags of window row k form one 64-bit word.  tail[lane]: when
+// the first window record continues the brick of the last front record, the
 // number of front records since that brick's entry (at most 22, the longest
 // crossing of a brick), else 0.
 __global__ __launch_bounds__(256) void k_brick_starts(const FrontRec* __restrict__ front,
-                                                      const SkirtRec* __restrict__ skirt,
                                                       const RayRec* __restrict__ lanes,
-                                                      const uint32_t* __restrict__ len_s,
                                                       const uint32_t* __restrict__ len_w, uint32_t nslices,
-                                                      const uint2* __restrict__ inc, uint32_t base_s,
+                                                      const uint2* __restrict__ inc, uint32_t base_w,
                                                       uint64_t* __restrict__ bstart, uint8_t* __restrict__ tail) {
   const uint32_t t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (t >= nslices) return;  // uniform per wavefront
   const uint32_t l = threadIdx.x & 63u, ray = t * kSlice + l;
   const FrontRec f = front[ray];
-  const SkirtRec sk = skirt[ray];
   const RayRec r = lanes[ray];
+  const uint32_t sw = __builtin_amdgcn_readfirstlane(r.off_w - l);  // the slice's window region
+  const uint32_t row0 = (sw - base_w) / kSlice;
+  const uint32_t lw = len_w[t];
   const uint32_t last = f.nf ? inc[f.off + (size_t)(f.nf - 1) * kSlice].x : kGapVox;
-  uint32_t prev = last;  // the record before the row
-  auto rows = [&](uint32_t off, uint32_t n, uint32_t len) {
-    const uint32_t sw = __builtin_amdgcn_readfirstlane(off - l);  // the slice's region
-    const uint32_t row0 = (sw - base_s) / kSlice;
-    for (uint32_t k = 0; k < len; ++k) {  // padding records are gap records
-      const uint32_t cur = inc[sw + (size_t)k * kSlice + l].x;
-      const bool bs = cur != kGapVox && (prev == kGapVox || (prev >> kBrickLog * 3) != (cur >> kBrickLog * 3));
-      const unsigned long long m = __ballot(bs);
-      if (l == 0) bstart[row0 + k] = m;
-      if (k < n) prev = cur;
-    }
-  };
-  rows(sk.off, sk.n, len_s[t]);
-  rows(r.off_w, r.nw, len_w[t]);
+  uint32_t prev = last;
+  for (uint32_t k = 0; k < lw; ++k) {  // padding records are gap records
+    const uint32_t cur = inc[sw + (size_t)k * kSlice + l].x;
+    const bool bs = cur != kGapVox && (prev == kGapVox || (prev >> kBrickLog * 3) != (cur >> kBrickLog * 3));
+    const unsigned long long m = __ballot(bs);
+    if (l == 0) bstart[row0 + k] = m;
+    prev = cur;
+  }
   uint32_t tl = 0;
-  if (f.nf && (sk.n || r.nw)) {
-    const uint32_t w0 = sk.n ? inc[sk.off].x : inc[r.off_w].x;
+  if (f.nf && r.nw) {
+    const uint32_t w0 = inc[sw + l].x;
     if (w0 != kGapVox && last != kGapVox && (w0 >> kBrickLog * 3) == (last >> kBrickLog * 3)) {
       uint32_t k = f.nf - 1;
       while (k > 0) {
@@ -671,11 +681,10 @@ __device__ __forceinline__ void win_pass1(const WinRay& r, uint32_t k0, uint32_t
 // memory traffic): 190 us either way.
 constexpr float kFtzMin = 0x1p-126f;
 
-// SKIRT: skirt records, over which the carried visibility sum kC goes on too.
-template <int UW, bool CS, bool SKIRT>
+template <int UW, bool CS>
 __device__ __forceinline__ void win_pass1_bl(const WinRay& r, uint32_t k0, uint32_t nw, const float (&ln)[UW],
                                              const float (&x)[UW], const uint64_t* __restrict__ bsw, Kahan& kL,
-                                             Kahan& kC, Kahan& kS, float& T, uint64_t& nz) {
+                                             Kahan& kS, float& T, uint64_t& nz) {
   uint64_t w[UW];
 #pragma unroll
   for (int u = 0; u < UW; ++u) w[u] = bsw[k0 + u];
@@ -697,7 +706,6 @@ __device__ __forceinline__ void win_pass1_bl(const WinRay& r, uint32_t k0, uint3
     const uint64_t counted = valid & __ballot(fminf(fminf(ap, ps), fminf(b, b * ps)) >= kFtzMin);
     T += __builtin_amdgcn_inverse_ballot_w64(counted) ? (V * ps) * (1.0f - nn) : 0.0f;
     nz |= counted;
-    if constexpr (SKIRT) kC.add(a);
     kL.add(a);  // a = 0 and l = 0 past the lane's last record: no select needed
     kS.add(ln[u]);
   }
@@ -708,7 +716,7 @@ __device__ __forceinline__ void win_pass1_any(const WinRay& r, uint32_t k0, uint
                                               const float (&x)[UW], const uint64_t* __restrict__ bsw, Kahan& kL,
                                               Kahan& kS, float& T, uint64_t& nz) {
   if constexpr (BL)
-    win_pass1_bl<UW, CS, false>(r, k0, nw, ln, x, bsw, kL, kL, kS, T, nz);
+    win_pass1_bl<UW, CS>(r, k0, nw, ln, x, bsw, kL, kS, T, nz);
   else
     win_pass1<UW, CS>(r, k0, nw, ln, x, kL, kS, T);
 }
@@ -745,8 +753,6 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
                                                     typename Msg<MO>::T* __restrict__ Xo,
                                                     const float* __restrict__ sigt, const float* __restrict__ biat,
                                                     int lookup_n, const FrontRec* __restrict__ front,
-                                                    const SkirtRec* __restrict__ skirt,
-                                                    const uint32_t* __restrict__ len_s, uint32_t base_s,
                                                     const uint64_t* __restrict__ bstart,
                                                     const uint8_t* __restrict__ tail) {
   typedef typename Msg<MI>::T TI;
@@ -786,7 +792,7 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
   r.z0 = rec.z0;
   r.inv = rec.inv_norm;
   r.d = rec.depth;
-  Kahan L0 = kL, S0 = kS;  // visibility and length sums at the window's start
+  const Kahan L0 = kL, S0 = kS;
   // the slice's window region (record k of lane l at sw + k * 64 + l), wave-uniform
   const uint32_t sw = __builtin_amdgcn_readfirstlane(rec.off_w - l);
   const uint32_t lws = __builtin_amdgcn_readfirstlane(lw);
@@ -802,11 +808,12 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
   uint64_t nz = 0;
   const uint64_t* bsw = nullptr;
   if constexpr (BL) {
-    // the pre pass enters the skirt (or, without one, the window) with the
-    // visibility sum of the front records in its first record's brick (every
-    // front tau is 0), at most 22 records, the longest crossing of a brick: 8
-    // record loads, then their 8 gathers, in flight at a time, summed in
-    // record order
+    // the pre pass enters the window with the visibility sum of the front
+    // records in the first window record's brick (every front tau is 0);
+    // bit l of word k of bsw: window record k of this lane enters a brick
+    // (the slice's rows of the word array, padded past the last slice)
+    // (at most 22 records, the longest crossing of a brick; 8 record loads,
+    // then their 8 gathers, in flight at a time, summed in record order)
     const FrontRec fr = front[ray];
     const uint32_t tl = tail[ray];
     const uint2* __restrict__ tr = inc + fr.off + (size_t)(fr.nf - tl) * kSlice;
@@ -823,31 +830,7 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
         if (b + i < tl) kp.add(__uint_as_float(et[i].y) * tx[i]);
     }
     kL = kp;
-    // the skirt: pass 1 only, the visibility carried along the ray (L0) goes
-    // on beside the restarted one; bit l of word k of bsw: record k of this
-    // lane enters a brick (the slice's rows, padded past the last slice)
-    const SkirtRec sk = skirt[ray];
-    const uint32_t lss = __builtin_amdgcn_readfirstlane(len_s[t]);
-    if (lss) {
-      const uint32_t ss = __builtin_amdgcn_readfirstlane(sk.off - l);
-      const Rsrc rs = make_rsrc(inc + ss, lss * kSlice * 8u);
-      bsw = bstart + (ss - base_s) / kSlice;
-      win_load<UW>(rs, lr, 0, e);
-      win_issue<MI, UW>(rx, e, lA, xA);
-      win_load<UW>(rs, lr, UW, e);
-      for (uint32_t k0 = 0;; k0 += 2 * UW) {
-        win_issue<MI, UW>(rx, e, lB, xB);
-        win_load<UW>(rs, lr, k0 + 2 * UW, e);
-        win_pass1_bl<UW, CS, true>(r, k0, sk.n, lA, xA, bsw, kL, L0, kS, T, nz);
-        if (k0 + UW >= lss) break;
-        win_issue<MI, UW>(rx, e, lA, xA);
-        win_load<UW>(rs, lr, k0 + 3 * UW, e);
-        win_pass1_bl<UW, CS, true>(r, k0 + UW, sk.n, lB, xB, bsw, kL, L0, kS, T, nz);
-        if (k0 + 2 * UW >= lss) break;
-      }
-      S0 = kS;
-    }
-    bsw = bstart + (sw - base_s) / kSlice;
+    bsw = bstart + (sw - base_w) / kSlice;
   }
   win_load<UW>(rr, lr, 0, e);
   win_issue<MI, UW>(rx, e, lA, xA);
@@ -1329,8 +1312,7 @@ void launch_ray_t(const CamPass& a, hipStream_t s, int part) {
   auto* k = a.brick_local ? (a.const_model ? k_ray_window<MI, MO, UW, true, true> : k_ray_window<MI, MO, UW, true, false>)
                           : (a.const_model ? k_ray_window<MI, MO, UW, false, true> : k_ray_window<MI, MO, UW, false, false>);
   hipLaunchKernelGGL(k, dim3(nb), dim3(64), 0, s, a.lanes, a.len_w, a.nslices, a.chunk_off, a.partial, a.inc, a.base_w,
-                     Xi, a.npairs, (typename Msg<MO>::T*)a.Xo, a.sig, a.bia, a.lookup_n, a.front, a.skirt, a.len_s, a.base_s,
-                     a.bstart, a.tail);
+                     Xi, a.npairs, (typename Msg<MO>::T*)a.Xo, a.sig, a.bia, a.lookup_n, a.front, a.bstart, a.tail);
 }
 
 template <int MI, int MO>
@@ -1385,23 +1367,21 @@ void launch_epilogue(const CamPass& a, hipStream_t s, int part) {
                      a.npairs, a.wseg_off, a.S, a.pl_v, a.pf_v, a.mid, out_scale, a.B, a.M, a.upd, a.all_pairs);
 }
 
-void launch_reslice(FrontRec* front, SkirtRec* skirt, RayRec* lanes, uint32_t npix, const uint2* sell,
-                    const int32_t* slot, const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_s,
-                    const uint32_t* len_s, uint32_t base_s, const uint32_t* off_w, const uint32_t* len_w,
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const int32_t* slot,
+                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
                     uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, unsigned long long* counts,
                     hipStream_t s) {
   if (npix == 0) return;
   auto* k = slot ? k_reslice<true> : k_reslice<false>;
-  hipLaunchKernelGGL(k, dim3(grid_for(npix, 256)), dim3(256), 0, s, front, skirt, lanes, npix, sell, slot, off_f, len_f,
-                     off_s, len_s, base_s, off_w, len_w, base_w, inc, any, wany, counts);
+  hipLaunchKernelGGL(k, dim3(grid_for(npix, 256)), dim3(256), 0, s, front, lanes, npix, sell, slot, off_f, len_f, off_w,
+                     len_w, base_w, inc, any, wany, counts);
 }
 
-void launch_brick_starts(const FrontRec* front, const SkirtRec* skirt, const RayRec* lanes, const uint32_t* len_s,
-                         const uint32_t* len_w, uint32_t nslices, const uint2* inc, uint32_t base_s, uint64_t* bstart,
-                         uint8_t* tail, hipStream_t s) {
+void launch_brick_starts(const FrontRec* front, const RayRec* lanes, const uint32_t* len_w, uint32_t nslices,
+                         const uint2* inc, uint32_t base_w, uint64_t* bstart, uint8_t* tail, hipStream_t s) {
   if (nslices == 0) return;
-  hipLaunchKernelGGL(k_brick_starts, dim3(grid_for(nslices, 4)), dim3(256), 0, s, front, skirt, lanes, len_s, len_w,
-                     nslices, inc, base_s, bstart, tail);
+  hipLaunchKernelGGL(k_brick_starts, dim3(grid_for(nslices, 4)), dim3(256), 0, s, front, lanes, len_w, nslices, inc,
+                     base_w, bstart, tail);
 }
 
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s) {

@@ -64,11 +64,9 @@ constexpr uint32_t kSlice = 64;           // rays per slice (one 8x8 pixel tile,
 
 // Per-ray records of one camera's traversal (one per lane of a slice).  A
 // ray's records are split into a front part, where the depth likelihood
-// psi(s) is exactly 0 in FP32, a skirt, where it is too small to lift a
-// message, and a window part; each part is a sliced-ELL region of its own:
-// front record k at FrontRec::off + k * kSlice, skirt record k (record nf + k
-// of the ray) at SkirtRec::off + k * kSlice, window record k (record nf + n +
-// k) at RayRec::off_w + k * kSlice.
+// psi(s) is exactly 0 in FP32, and a window part; each part is a sliced-ELL
+// region of its own: front record k at FrontRec::off + k * kSlice, window
+// record k (record nf + k of the ray) at RayRec::off_w + k * kSlice.
 struct FrontRec {
   uint32_t off;        // first front record
   uint32_t nf;         // front records (voxels + gap records)
@@ -82,12 +80,6 @@ struct RayRec {
   uint32_t cell_flags; // sensor-model lookup offset (bits 0..29) | kInfTerm | kRanOut
   float ks, kc;        // Kahan sum of the front chord lengths (sum, compensation)
 };
-// The skirt of a ray, between its front and its window (kSkirtU): record k at
-// off + k * kSlice.
-struct SkirtRec {
-  uint32_t off;        // first skirt record
-  uint32_t n;          // skirt records
-};
 constexpr uint32_t kChunk = 16;  // front records per lane in one chunk of the front kernel
 
 // A record belongs to the front while d - (s + bias(s)) > kFrontU * 3 sigma(s)
@@ -100,18 +92,6 @@ constexpr uint32_t kChunk = 16;  // front records per lane in one chunk of the f
 // reference's flush-to-zero arithmetic such a tau is exactly 0 (its factor
 // 0.398942 exp(-u^2/2) is below 2^-126 from u = 13.15 on).
 constexpr float kFrontU = 13.5f;
-// Past the front, while d - (s + bias(s)) > kSkirtU * 3 sigma(s), psi is below
-// 0.4 e^{-47.5} / (3 sigma) < 3.1e-19 for any sigma above 1 mm.  A message
-// leaves the clamp floor F_EPS l only if mu1 > F_EPS * 1e-7 = 1e-11, which
-// these records cannot reach, and what they add to a later P (about one such
-// psi, the sum growing tenfold from record to record) is below the FP32
-// rounding of any P that does.  So their messages are the constant F_EPS l,
-// like the front's, and P starts after them.  Their taus still decide where
-// the brick-local pre pass stops restarting, and they are summed into T: the
-// skirt is the part of the ray that only pass 1 reads.  With the visibility
-// carried along the ray there is nothing to decide and the front reaches up
-// to kSkirtU.
-constexpr float kSkirtU = 9.75f;
 constexpr uint32_t kRanOut = 0x80000000u;  // ray left the active space before truncation
 // the ray ran out and its depth lies beyond the exit: the infinity term applies
 // (gvdbkernels.cu:1196-1208), decided in FP64 from the exact exit depth

@@ -35,18 +35,17 @@ void launch_slice_len(const uint32_t* counts, uint32_t ntiles, uint32_t* slice_l
                       hipStream_t s);
 // sliced-ELL emission: record k of lane l of slice t at slice_off[t] + k*64 + l
 // for k below the ray's record count (nothing past it is written), split
-// into front, skirt and window: front[t*64+l].nf front records, then
-// skirt[t*64+l].n skirt records (none with u_front = kSkirtU), then
+// into front and window: front[t*64+l].nf front records, then
 // lanes[t*64+l].nw window records (the ray's description, the Kahan state of
-// the front's length sum); cnt_f / cnt_s / cnt_w the same per tiled pixel.  A ray
+// the front's length sum); cnt_f / cnt_w the same per tiled pixel.  A ray
 // with more records than its slice's length slice_len[t] (sized by a count
 // or a bound of it) sets *overflow.  all_active (full-ray activation, fewer
 // than 2^23 bricks in the grid): the records hold (linear brick index) * 512
 // + voxel instead of pool ids.
 void launch_emit(const CamGeom& c, const GridGeom& g, const float* depth, const float* sig, const float* bia,
                  const int32_t* slot, const uint32_t* slice_off, const uint32_t* slice_len, uint2* sell,
-                 FrontRec* front, SkirtRec* skirt, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_s, uint32_t* cnt_w,
-                 float u_front, uint32_t* overflow, bool all_active, hipStream_t s);
+                 FrontRec* front, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_w, uint32_t* overflow,
+                 bool all_active, hipStream_t s);
 
 // map evaluation of one camera's pixels (log-likelihood, expected depth,
 // accuracy and simple accuracy images in row-major pixel order, any may be
@@ -127,11 +126,8 @@ struct CamPass {
   const RayRec* lanes;     // one per lane of every slice
   const uint32_t* len_f;   // front records per lane of each slice
   const uint32_t* len_w;   // window records per lane of each slice
-  const SkirtRec* skirt;   // one per lane of every slice (brick_local)
-  const uint32_t* len_s;   // skirt records per lane of each slice
-  uint32_t base_s;         // first record of the skirt region
   uint32_t nslices;
-  const uint2* inc;        // sliced records {pair | kGapVox, chord length}: front, skirt and window regions
+  const uint2* inc;        // sliced records {pair | kGapVox, chord length}: front region, then window region
   const uint32_t* win_idx; // per window position (voxel order): its record's slot in the window region
   uint32_t base_w;         // first record of the window region
   const uint32_t* chunk_off;   // nslices + 1: first front chunk of each slice
@@ -177,34 +173,30 @@ struct CamPass {
   int msg_type;
   int ray_sched;           // RaySched
   // pre-pass visibility restarted at brick entries until a tau survives
-  // flush-to-zero (MRF_VIS_BRICK_LOCAL): per skirt and window row of every
-  // slice the lanes whose record enters a brick, and per lane the front
-  // records that share the brick of the first record after them
+  // flush-to-zero (MRF_VIS_BRICK_LOCAL): per window row of every slice the
+  // lanes whose record enters a brick, and per lane the front records that
+  // share the first window record's brick
   bool brick_local;
   const uint64_t* bstart;
   const uint8_t* tail;
 };
-// copy into the final front, skirt and window regions (the skirt region at
-// base_s, the window region at base_w).
+// copy into the final front/window regions; window region starts at base_w.
 // any / wany: pool-sized byte flags of voxels touched by a live / window
 // record (set, never cleared); counts[0] / counts[1] += the live / live
 // window records, counts[2] += all records (gap records included),
 // counts[3] += rays with records
 // slot (may be null): the staged records hold (linear brick index) * 512 +
 // voxel and become pool ids through it
-void launch_reslice(FrontRec* front, SkirtRec* skirt, RayRec* lanes, uint32_t npix, const uint2* sell,
-                    const int32_t* slot, const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_s,
-                    const uint32_t* len_s, uint32_t base_s, const uint32_t* off_w, const uint32_t* len_w,
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const int32_t* slot,
+                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
                     uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, unsigned long long* counts, hipStream_t s);
-// brick entries of every skirt and window record (records still hold voxel
-// ids): bstart[row, counted from the skirt region's first] bit l = the record
-// of lane l in that row enters a brick (the ray's first record, the record
-// after a gap, or a voxel in another brick than the previous record's);
-// tail[lane] = front records at the end of the front that lie in the brick of
-// the first record after it
-void launch_brick_starts(const FrontRec* front, const SkirtRec* skirt, const RayRec* lanes, const uint32_t* len_s,
-                         const uint32_t* len_w, uint32_t nslices, const uint2* inc, uint32_t base_s, uint64_t* bstart,
-                         uint8_t* tail, hipStream_t s);
+// brick entries of every window record (records still hold voxel ids):
+// bstart[(region row of the slice) + k] bit l = record k of lane l enters a
+// brick (the ray's first record, the record after a gap, or a voxel in
+// another brick than the previous record's); tail[lane] = front records at
+// the end of the front that lie in the first window record's brick
+void launch_brick_starts(const FrontRec* front, const RayRec* lanes, const uint32_t* len_w, uint32_t nslices,
+                         const uint2* inc, uint32_t base_w, uint64_t* bstart, uint8_t* tail, hipStream_t s);
 // front chunks per slice (cnt has nslices + 1 entries, the last 0), the
 // descriptor of every chunk from their offsets, and the per-lane front spans
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s);

@@ -169,34 +169,24 @@ __device__ __forceinline__ bool ray_entry(const GridGeom& g, const RaySetup& rs,
   return true;
 }
 
-// Front/skirt/window split of one ray during its emission, with the ray
-// kernel's own FP32 depth sums: a part ends at the first record whose exit
-// depth s has d - (s + bias(s)) <= u * 3 sigma(s), u = u_front for the front
-// (kSkirtU where there is no skirt) and kSkirtU for the skirt.  The Kahan
-// state of the front's length sum is kept: the parts after it continue it.
+// Front/window split of one ray during its emission, with the ray kernel's
+// own FP32 depth sums: the front ends at the first record whose exit depth s
+// has d - (s + bias(s)) <= kFrontU * 3 sigma(s).  The Kahan state of the
+// front's length sum is kept: the window continues it.
 struct FrontSplit {
   Poly sig, bia;
-  float z0, inv_norm, depth, u;
-  Kahan kS, kF;
-  uint32_t nf, w0;  // the first record past the front, the first window record (once their part has ended)
-  int part;         // 0 front, 1 skirt, 2 window
+  float z0, inv_norm, depth;
+  Kahan kS;
+  uint32_t nf;  // the first window record (valid once open is false)
+  bool open;
   __device__ __forceinline__ void record(uint32_t k, float ln) {
-    if (part == 2) return;
+    if (!open) return;
     const float s = z0 + kS.at(ln) * inv_norm;
     const float sg = sig(s);
-    const float left = depth - (s + bia(s)), w3 = 3.0f * sg;
-    if (!(sg > 0.0f && left > u * w3)) {
-      if (part == 0) {
-        nf = k;
-        kF = kS;
-        part = 1;
-        u = kSkirtU;
-      }
-      if (!(sg > 0.0f && left > kSkirtU * w3)) {
-        w0 = k;
-        part = 2;
-        return;
-      }
+    if (!(sg > 0.0f && depth - (s + bia(s)) > kFrontU * (3.0f * sg))) {
+      nf = k;
+      open = false;
+      return;
     }
     kS.add(ln);
   }
@@ -311,7 +301,7 @@ __device__ __forceinline__ Steps<F64> first_crossings(const RaySetup& rs, const 
 // Records of one ray are written out[0], out[kSlice], out[2 kSlice], ...
 // (record k of the 64 rays of a pixel tile is contiguous: sliced ELL), the
 // first cap of them (the count goes on past cap); vis, when given, splits
-// them into front, skirt and window (vis->record(k, chord) per record in order,
+// them into front and window (vis->record(k, chord) per record in order,
 // vis->z0 the planar depth at the entry of the first).  kEmit looks each
 // brick's slot up and writes the voxels' pool ids; kEmitAll needs no look-up
 // and writes (linear brick index) * 512 + voxel, so that its loop holds no
@@ -606,26 +596,23 @@ __global__ void k_slice_len(const uint32_t* __restrict__ counts, uint32_t ntiles
   }
 }
 
-// Emission of every ray's records into the staging lists, split into front,
-// skirt and window as they go: front[pix].nf front records, then
-// skirt[pix].n skirt and lanes[pix].nw window records; cnt_f / cnt_s / cnt_w
-// per tiled pixel.
+// Emission of every ray's records into the staging lists, split into front
+// and window as they go: front[pix].nf front records, then lanes[pix].nw
+// window records; cnt_f / cnt_w per tiled pixel.
 template <bool F64, bool ALL>
 __global__ void k_emit(CamGeom c, GridGeom g, const float* __restrict__ depth, const float* __restrict__ sig,
                        const float* __restrict__ bia, const int32_t* __restrict__ slot,
                        const uint32_t* __restrict__ slice_off, const uint32_t* __restrict__ slice_len,
-                       uint2* __restrict__ sell, FrontRec* __restrict__ front, SkirtRec* __restrict__ skirt,
-                       RayRec* __restrict__ lanes, uint32_t* __restrict__ cnt_f, uint32_t* __restrict__ cnt_s,
-                       uint32_t* __restrict__ cnt_w, float u_front, uint32_t* __restrict__ overflow) {
+                       uint2* __restrict__ sell, FrontRec* __restrict__ front, RayRec* __restrict__ lanes,
+                       uint32_t* __restrict__ cnt_f, uint32_t* __restrict__ cnt_w, uint32_t* __restrict__ overflow) {
   const int pix = blockIdx.x * blockDim.x + threadIdx.x;
   if (pix >= tiled_pixels(c)) return;
   const uint32_t tile = (uint32_t)pix >> 6, lane = (uint32_t)pix & 63u;
   uint2* out = sell + slice_off[tile] + lane;
   PixelCtx p = load_pixel(c, g, depth, pix);
   FrontRec f;
-  f.off = slice_off[tile] + lane;  // the parts follow each other until the reslice
+  f.off = slice_off[tile] + lane;  // front and window records follow each other until the reslice
   f.nf = 0;
-  SkirtRec sk = {0u, 0u};
   RayRec r;
   r.off_w = 0;
   r.nw = 0;
@@ -641,10 +628,9 @@ __global__ void k_emit(CamGeom c, GridGeom g, const float* __restrict__ depth, c
     sp.inv_norm = (float)(1.0 / p.rs.norm);
     sp.depth = p.d;
     sp.z0 = 0.0f;
-    sp.kS = sp.kF = {0.0f, 0.0f};
-    sp.nf = sp.w0 = 0;
-    sp.part = 0;
-    sp.u = u_front;
+    sp.kS = {0.0f, 0.0f};
+    sp.nf = 0;
+    sp.open = true;
     const uint32_t cap = slice_len[tile];
     const Truncation trunc = truncation(g, p, sig, bia);
     WalkOut wo = walk<ALL ? kEmitAll : kEmit, F64>(g, p.rs, trunc, slot, out, cap, &sp);
@@ -653,13 +639,11 @@ __global__ void k_emit(CamGeom c, GridGeom g, const float* __restrict__ depth, c
       atomicOr(overflow, 1u);
       n = cap;
     }
-    const uint32_t nf = sp.part == 0 ? n : min(sp.nf, n), w0 = sp.part < 2 ? n : min(sp.w0, n);
-    if (sp.part == 0) sp.kF = sp.kS;
+    const uint32_t nf = sp.open ? n : min(sp.nf, n);
     f.nf = nf;
-    sk.n = w0 - nf;
-    r.nw = n - w0;
-    r.ks = sp.kF.s;
-    r.kc = sp.kF.c;
+    r.nw = n - nf;
+    r.ks = sp.kS.s;
+    r.kc = sp.kS.c;
     r.z0 = wo.z0;
     r.inv_norm = sp.inv_norm;
     r.depth = p.d;
@@ -671,10 +655,8 @@ __global__ void k_emit(CamGeom c, GridGeom g, const float* __restrict__ depth, c
   }
   // records past the ray's own are never read: no padding
   front[pix] = f;
-  skirt[pix] = sk;
   lanes[pix] = r;
   cnt_f[pix] = f.nf;
-  cnt_s[pix] = sk.n;
   cnt_w[pix] = r.nw;
 }
 
@@ -963,14 +945,14 @@ void launch_slice_len(const uint32_t* counts, uint32_t ntiles, uint32_t* slice_l
 
 void launch_emit(const CamGeom& c, const GridGeom& g, const float* depth, const float* sig, const float* bia,
                  const int32_t* slot, const uint32_t* slice_off, const uint32_t* slice_len, uint2* sell,
-                 FrontRec* front, SkirtRec* skirt, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_s, uint32_t* cnt_w,
-                 float u_front, uint32_t* overflow, bool all_active, hipStream_t s) {
+                 FrontRec* front, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_w, uint32_t* overflow,
+                 bool all_active, hipStream_t s) {
   const int n = tiled_pixels(c);
   const bool f64 = dda_fits_f64(c, g);
   auto* k = all_active ? (f64 ? k_emit<true, true> : k_emit<false, true>)
                        : (f64 ? k_emit<true, false> : k_emit<false, false>);
   hipLaunchKernelGGL(k, dim3((n + 127) / 128), dim3(128), 0, s, c, g, depth, sig, bia, slot, slice_off, slice_len, sell,
-                     front, skirt, lanes, cnt_f, cnt_s, cnt_w, u_front, overflow);
+                     front, lanes, cnt_f, cnt_w, overflow);
 }
 
 }  // namespace mrf
