@@ -710,19 +710,17 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   // (any and wany are all zero here: cleared before the first camera, and
   // behind by the pair table of each camera)
   HIPCHK(c, hipMemsetAsync(c->d_total + 2, 0, 32, s));
-  launch_reslice(cam.d_front, cam.d_lanes, (uint32_t)npix, c->d_sell0, all_active ? c->d_slot : nullptr, c->d_offs,
-                 cam.d_len_f, c->d_has, cam.d_len_w, (uint32_t)nrec_f, cam.d_inc, any, wany,
-                 (unsigned long long*)(c->d_total + 2), s);
   if (c->p.brick_local_vis == MRF_VIS_BRICK_LOCAL) {
-    // brick entries of the window records, while the records hold voxel ids;
-    // rows past the last slice read as zero words (the window kernel's
-    // batches may look up to 16 rows past a slice's longest ray)
+    // brick entries of the window records; rows past the last slice read as
+    // zero words (the window kernel's batches may look up to 16 rows past a
+    // slice's longest ray)
     const size_t wrows = (size_t)(nrec_w / kSlice);
     if ((rc = dalloc(c, &cam.d_bstart, wrows + 32)) || (rc = dalloc(c, &cam.d_tail, npix))) return rc;
     launch_zero_words(cam.d_bstart + wrows, 32 * sizeof(uint64_t), s);
-    launch_brick_starts(cam.d_front, cam.d_lanes, cam.d_len_w, ntiles, cam.d_inc, (uint32_t)nrec_f, cam.d_bstart,
-                        cam.d_tail, s);
   }
+  launch_reslice(cam.d_front, cam.d_lanes, ntiles, c->d_sell0, all_active ? c->d_slot : nullptr, c->d_offs, cam.d_len_f,
+                 c->d_has, cam.d_len_w, (uint32_t)nrec_f, cam.d_inc, any, wany, cam.d_bstart, cam.d_tail,
+                 (unsigned long long*)(c->d_total + 2), s);
   // one allocation for the partial sums, the static sums and the masks of
   // changing records (per chunk and lane each)
   const size_t nparts = (size_t)cam.nchunks * kSlice;

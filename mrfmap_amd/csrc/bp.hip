@@ -151,29 +151,44 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 // ---------------------------------------------------------------- list layout
 // Copy every ray's records into the front and window regions of the final
 // record buffer (sliced: lane l of slice t at region offset + k * 64 + l),
-// padding each lane to its slice's length with gap records.  One wavefront
-// is one slice, so record k of the 64 rays moves together: per row the
-// voxel flags any[v] = 1 (every live record) and wany[v] = 1 (live window
-// records) are set, skipping a lane whose voxel equals that of the ray to
-// its left or above in the pixel tile (the flags say only whether), and
-// counts[0] / counts[1] gain the row's live / live window records; per
-// wavefront counts[2] gains its rays' records (gap records included) and
-// counts[3] its rays with records.
+// padding each lane to its slice's length with gap records.  Record k of the
+// 64 rays of a slice moves together: per row the voxel flags any[v] = 1
+// (every live record) and wany[v] = 1 (live window records) are set, skipping
+// a lane whose voxel equals that of the ray to its left or above in the pixel
+// tile (the flags say only whether), and counts[0] / counts[1] gain the row's
+// live / live window records; counts[2] gains the slice's records (gap
+// records included) and counts[3] its rays with records.
 // SLOTS: the staged records hold (linear brick index) * 512 + voxel, and the
 // brick's slot is looked up here (neighbouring rays share their bricks).
+//
+// Brick entries of the window records (bstart; null when not wanted): record
+// k of lane l enters a brick when it is a voxel record and the previous
+// record of its ray is a gap record, lies in another brick, or does not
+// exist.  The 64 lanes' flags of a window row form one 64-bit word.
+// tail[lane]: when the first window record continues the brick of the last
+// front record, the number of front records since that brick's entry (at most
+// 22, the longest crossing of a brick), else 0.  Both look one record back,
+// at the staged copy.
+//
+// A block of four waves is one slice, batches of kB rows going to its waves
+// in turn: a wave's batch is a chain of loads (record, slot) before its
+// stores, and one wave per slice leaves four waves per SIMD at 640x480 and
+// fewer than one below 160x120.  640x480 at 1 cm, 161 M records, 2.6 GB read
+// and written: 795 us; one wave per slice and the brick entries as a pass of
+// their own took 869 + 116 us (160x120 at 4 cm: 30 us against 38 + 54).
 template <bool SLOTS>
 __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, RayRec* __restrict__ lanes,
-                                                 uint32_t npix, const uint2* __restrict__ sell,
-                                                 const int32_t* __restrict__ slot,
+                                                 const uint2* __restrict__ sell, const int32_t* __restrict__ slot,
                                                  const uint32_t* __restrict__ off_f, const uint32_t* __restrict__ len_f,
                                                  const uint32_t* __restrict__ off_w, const uint32_t* __restrict__ len_w,
                                                  uint32_t base_w, uint2* __restrict__ inc, uint8_t* __restrict__ any,
-                                                 uint8_t* __restrict__ wany, unsigned long long* __restrict__ counts) {
-  const uint32_t ray = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ray >= npix) return;  // uniform per wavefront: npix is a multiple of 64
-  const uint32_t t = ray >> 6, l = ray & 63u;
+                                                 uint8_t* __restrict__ wany, uint64_t* __restrict__ bstart,
+                                                 uint8_t* __restrict__ tail, unsigned long long* __restrict__ counts) {
+  constexpr uint32_t kW = 4, kB = 8;
+  __shared__ uint64_t wave_counts[kW][2];
+  const uint32_t t = blockIdx.x, wave = threadIdx.x >> 6, l = threadIdx.x & 63u, ray = t * kSlice + l;
   const FrontRec f = front[ray];
-  const uint32_t rnw = lanes[ray].nw;
+  const uint32_t rnw = lanes[ray].nw, nr = f.nf + rnw;
   const uint2* __restrict__ src = sell + f.off;
   const uint32_t fo = off_f[t] + l, wo = base_w + off_w[t] + l;
   const uint2 gap = make_uint2(kGapVox, 0u);
@@ -182,10 +197,8 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
     const uint32_t left = (uint32_t)__shfl_up((int)v, 1, 64), up = (uint32_t)__shfl_up((int)v, 8, 64);
     return ((l & 7u) != 0u && left == v) || (l >= 8u && up == v);
   };
-  // rows in batches of kB: the batch's loads are in flight together (the
-  // bounds lf, lw are uniform per wavefront, so every lane takes part in the
-  // shuffles)
-  constexpr uint32_t kB = 8;
+  // a batch's loads are in flight together (the bounds lf, lw are uniform per
+  // wavefront, so every lane takes part in the shuffles)
   auto pool_ids = [&](uint2(&e)[kB]) {
     if constexpr (SLOTS) {
       int32_t sl[kB];
@@ -198,7 +211,7 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
   };
   uint64_t nl = 0, nw = 0;
   const uint32_t lf = len_f[t], lw = len_w[t];
-  for (uint32_t k0 = 0; k0 < lf; k0 += kB) {
+  for (uint32_t k0 = wave * kB; k0 < lf; k0 += kW * kB) {
     uint2 e[kB];
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
@@ -218,12 +231,26 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
     }
   }
   const uint2* __restrict__ srcw = src + (size_t)f.nf * kSlice;
-  for (uint32_t k0 = 0; k0 < lw; k0 += kB) {
+  for (uint32_t k0 = wave * kB; k0 < lw; k0 += kW * kB) {
     uint2 e[kB];
+    uint32_t prev = kGapVox;  // the ray's record before the batch
+    if (bstart && f.nf + k0 > 0 && k0 <= rnw) prev = src[(size_t)(f.nf + k0 - 1) * kSlice].x;
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
       e[u] = gap;
       if (k0 + u < rnw) e[u] = srcw[(size_t)(k0 + u) * kSlice];
+    }
+    if (bstart) {
+      uint64_t mine = 0;  // lane u: the word of row k0 + u
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u) {
+        const uint32_t cur = e[u].x;
+        const uint64_t m =
+            __ballot(cur != kGapVox && (prev == kGapVox || (prev >> kBrickLog * 3) != (cur >> kBrickLog * 3)));
+        if (l == u) mine = m;
+        prev = cur;
+      }
+      if (l < kB && k0 + l < lw) bstart[off_w[t] / kSlice + k0 + l] = mine;
     }
     pool_ids(e);
 #pragma unroll
@@ -242,64 +269,50 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
       }
     }
   }
-  // the ray's records (gap records included) and whether it has any
-  uint32_t nr = f.nf + rnw;
-  const uint64_t nray = (uint64_t)__popcll(__ballot(nr != 0u));
-  for (int o = 32; o > 0; o >>= 1) nr += (uint32_t)__shfl_xor((int)nr, o, 64);
-  if (l == 0) {
-    if (nl) atomicAdd(&counts[0], (unsigned long long)nl);
-    if (nw) atomicAdd(&counts[1], (unsigned long long)nw);
-    if (nr) atomicAdd(&counts[2], (unsigned long long)nr);
-    if (nray) atomicAdd(&counts[3], (unsigned long long)nray);
+  if (tail && wave == kW - 1) {  // the wave with the fewest batches
+    uint32_t tl = 0;
+    if (f.nf && rnw) {
+      const uint32_t w0 = srcw[0].x, last = src[(size_t)(f.nf - 1) * kSlice].x;
+      auto same = [&](uint32_t v) { return v != kGapVox && (v >> kBrickLog * 3) == (w0 >> kBrickLog * 3); };
+      if (w0 != kGapVox && same(last)) {
+        bool more = true;
+        for (tl = 1; more;) {  // records back from the last front record, kB at a time
+          uint32_t pv[kB];
+#pragma unroll
+          for (uint32_t u = 0; u < kB; ++u)
+            pv[u] = tl + u < f.nf ? src[(size_t)(f.nf - 1 - tl - u) * kSlice].x : kGapVox;
+#pragma unroll
+          for (uint32_t u = 0; u < kB; ++u) {
+            more = more && same(pv[u]);
+            if (more) ++tl;
+          }
+        }
+      }
+    }
+    tail[ray] = (uint8_t)tl;
   }
+  if (l == 0) {
+    wave_counts[wave][0] = nl;
+    wave_counts[wave][1] = nw;
+  }
+  __syncthreads();  // every wave has read the slice's descriptions as well
+  if (wave != 0) return;
   front[ray].off = fo;
   lanes[ray].off_w = wo;
-}
-
-// Brick entries of the window records, one wavefront per slice, while the
-// records still hold voxel ids (slot * 512 + voxel in the brick): record k
-// of lane l enters a brick when it is a voxel record and the previous record
-// of its ray is a gap record, lies in another slot, or does not exist.  The
-// 64 lanes' flags of window row k form one 64-bit word.  tail[lane]: when
-// the first window record continues the brick of the last front record, the
-// number of front records since that brick's entry (at most 22, the longest
-// crossing of a brick), else 0.
-__global__ __launch_bounds__(256) void k_brick_starts(const FrontRec* __restrict__ front,
-                                                      const RayRec* __restrict__ lanes,
-                                                      const uint32_t* __restrict__ len_w, uint32_t nslices,
-                                                      const uint2* __restrict__ inc, uint32_t base_w,
-                                                      uint64_t* __restrict__ bstart, uint8_t* __restrict__ tail) {
-  const uint32_t t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (t >= nslices) return;  // uniform per wavefront
-  const uint32_t l = threadIdx.x & 63u, ray = t * kSlice + l;
-  const FrontRec f = front[ray];
-  const RayRec r = lanes[ray];
-  const uint32_t sw = __builtin_amdgcn_readfirstlane(r.off_w - l);  // the slice's window region
-  const uint32_t row0 = (sw - base_w) / kSlice;
-  const uint32_t lw = len_w[t];
-  const uint32_t last = f.nf ? inc[f.off + (size_t)(f.nf - 1) * kSlice].x : kGapVox;
-  uint32_t prev = last;
-  for (uint32_t k = 0; k < lw; ++k) {  // padding records are gap records
-    const uint32_t cur = inc[sw + (size_t)k * kSlice + l].x;
-    const bool bs = cur != kGapVox && (prev == kGapVox || (prev >> kBrickLog * 3) != (cur >> kBrickLog * 3));
-    const unsigned long long m = __ballot(bs);
-    if (l == 0) bstart[row0 + k] = m;
-    prev = cur;
-  }
-  uint32_t tl = 0;
-  if (f.nf && r.nw) {
-    const uint32_t w0 = inc[sw + l].x;
-    if (w0 != kGapVox && last != kGapVox && (w0 >> kBrickLog * 3) == (last >> kBrickLog * 3)) {
-      uint32_t k = f.nf - 1;
-      while (k > 0) {
-        const uint32_t pv = inc[f.off + (size_t)(k - 1) * kSlice].x;
-        if (pv == kGapVox || (pv >> kBrickLog * 3) != (w0 >> kBrickLog * 3)) break;
-        --k;
-      }
-      tl = f.nf - k;
+  // the slice's records (gap records included) and its rays with any
+  const uint64_t nray = (uint64_t)__popcll(__ballot(nr != 0u));
+  uint32_t nrec = nr;
+  for (int o = 32; o > 0; o >>= 1) nrec += (uint32_t)__shfl_xor((int)nrec, o, 64);
+  if (l == 0) {
+    for (uint32_t w = 1; w < kW; ++w) {
+      nl += wave_counts[w][0];
+      nw += wave_counts[w][1];
     }
+    if (nl) atomicAdd(&counts[0], (unsigned long long)nl);
+    if (nw) atomicAdd(&counts[1], (unsigned long long)nw);
+    if (nrec) atomicAdd(&counts[2], (unsigned long long)nrec);
+    if (nray) atomicAdd(&counts[3], (unsigned long long)nray);
   }
-  tail[ray] = (uint8_t)tl;
 }
 
 // Front chunks: a slice with window records needs ceil(len_f / kChunk) of
@@ -1367,21 +1380,14 @@ void launch_epilogue(const CamPass& a, hipStream_t s, int part) {
                      a.npairs, a.wseg_off, a.S, a.pl_v, a.pf_v, a.mid, out_scale, a.B, a.M, a.upd, a.all_pairs);
 }
 
-void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const int32_t* slot,
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t nslices, const uint2* sell, const int32_t* slot,
                     const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
-                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, unsigned long long* counts,
-                    hipStream_t s) {
-  if (npix == 0) return;
-  auto* k = slot ? k_reslice<true> : k_reslice<false>;
-  hipLaunchKernelGGL(k, dim3(grid_for(npix, 256)), dim3(256), 0, s, front, lanes, npix, sell, slot, off_f, len_f, off_w,
-                     len_w, base_w, inc, any, wany, counts);
-}
-
-void launch_brick_starts(const FrontRec* front, const RayRec* lanes, const uint32_t* len_w, uint32_t nslices,
-                         const uint2* inc, uint32_t base_w, uint64_t* bstart, uint8_t* tail, hipStream_t s) {
+                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail,
+                    unsigned long long* counts, hipStream_t s) {
   if (nslices == 0) return;
-  hipLaunchKernelGGL(k_brick_starts, dim3(grid_for(nslices, 4)), dim3(256), 0, s, front, lanes, len_w, nslices, inc,
-                     base_w, bstart, tail);
+  auto* k = slot ? k_reslice<true> : k_reslice<false>;
+  hipLaunchKernelGGL(k, dim3(nslices), dim3(256), 0, s, front, lanes, sell, slot, off_f, len_f, off_w, len_w, base_w, inc,
+                     any, wany, bstart, tail, counts);
 }
 
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s) {

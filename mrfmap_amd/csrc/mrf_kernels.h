@@ -187,16 +187,15 @@ struct CamPass {
 // counts[3] += rays with records
 // slot (may be null): the staged records hold (linear brick index) * 512 +
 // voxel and become pool ids through it
-void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t npix, const uint2* sell, const int32_t* slot,
-                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
-                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, unsigned long long* counts, hipStream_t s);
-// brick entries of every window record (records still hold voxel ids):
+// bstart / tail (both or neither null), brick entries of the window records:
 // bstart[(region row of the slice) + k] bit l = record k of lane l enters a
 // brick (the ray's first record, the record after a gap, or a voxel in
 // another brick than the previous record's); tail[lane] = front records at
 // the end of the front that lie in the first window record's brick
-void launch_brick_starts(const FrontRec* front, const RayRec* lanes, const uint32_t* len_w, uint32_t nslices,
-                         const uint2* inc, uint32_t base_w, uint64_t* bstart, uint8_t* tail, hipStream_t s);
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t nslices, const uint2* sell, const int32_t* slot,
+                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
+                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail,
+                    unsigned long long* counts, hipStream_t s);
 // front chunks per slice (cnt has nslices + 1 entries, the last 0), the
 // descriptor of every chunk from their offsets, and the per-lane front spans
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s);
