@@ -114,11 +114,10 @@ struct mrf_ctx {
   size_t cap_tiles = 0;
   // segment-build scratch (per record), per-pair scratch and the emitted lists
   uint32_t *d_keys_in = nullptr, *d_keys_out = nullptr, *d_vals_in = nullptr;  // window sort (values out: win_idx)
-  uint32_t *d_x0 = nullptr, *d_x1 = nullptr;  // window head flags and their scan
   size_t cap_sort = 0;
   uint32_t* d_vflag = nullptr;  // 4 pool-sized tables: touched, window-touched and their scans
   size_t cap_vflag = 0;
-  uint32_t* d_acc = nullptr;  // 6 words per pair: three 64-bit fixed-point chord-length sums
+  uint64_t* d_acc = nullptr;  // per pair three fixed-point chord-length sums
   size_t cap_acc = 0;
   uint2* d_sell0 = nullptr;
   size_t cap_sell0 = 0;
@@ -483,13 +482,11 @@ int ensure_sort(mrf_ctx* c, size_t n, int bits) {
   if (n > c->cap_sort) {
     n += n / 4;  // headroom: the next camera is likely a little larger, and a free waits for the device
     dfree(&c->d_keys_in); dfree(&c->d_keys_out); dfree(&c->d_vals_in);
-    dfree(&c->d_x0); dfree(&c->d_x1);
     c->cap_sort = 0;
     int rc;
     const size_t nx = n + 1024;
     if ((rc = dalloc(c, &c->d_keys_in, nx)) || (rc = dalloc(c, &c->d_keys_out, nx)) ||
-        (rc = dalloc(c, &c->d_vals_in, nx)) ||
-        (rc = dalloc(c, &c->d_x0, nx)) || (rc = dalloc(c, &c->d_x1, nx)))
+        (rc = dalloc(c, &c->d_vals_in, nx)))
       return rc;
     c->cap_sort = n;
   }
@@ -564,7 +561,7 @@ int ensure_acc(mrf_ctx* c, size_t np) {
   np += np / 4;
   dfree(&c->d_acc);
   c->cap_acc = 0;
-  int rc = dalloc(c, &c->d_acc, 6 * np);
+  int rc = dalloc(c, &c->d_acc, 3 * np);
   if (rc) return rc;
   c->cap_acc = np;
   return MRF_OK;
@@ -768,27 +765,20 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   if ((rc = dalloc(c, &cam.d_wseg_off, (size_t)nwp + 1)) ||
       (rc = dalloc(c, &cam.d_win_idx, std::max<uint64_t>(nrec_w, 1))))
     return rc;
-  uint32_t* acc_w = c->d_acc;
-  uint32_t* acc_f = c->d_acc + 2 * (size_t)np;
-  uint32_t* acc_r = c->d_acc + 4 * (size_t)np;
-  launch_pair_lengths(cam.d_inc, nrec, nrec_f, pid, acc_f, acc_r, np, c->d_keys_in, c->d_vals_in, nwp, s);
+  uint64_t* acc_w = c->d_acc;
+  uint64_t* acc_f = c->d_acc + (size_t)np;
+  uint64_t* acc_r = c->d_acc + 2 * (size_t)np;
+  launch_pair_lengths(cam.d_inc, nrec, nrec_f, pid, (uint32_t*)acc_f, (uint32_t*)acc_r, np, c->d_keys_in, c->d_vals_in, nwp, s);
   // 6. window segments: the window records stably sorted by pair
   HIPCHK(c, sort_window((uint32_t)nrec_w, wbits, c->d_keys_in, c->d_keys_out, c->d_vals_in, cam.d_win_idx,
                         c->d_sort_tmp, c->sort_tmp_bytes, s));
-  uint32_t* whead = c->d_x0;
-  uint32_t* hw = c->d_x1;
-  if (nwin) {
-    launch_window_heads(c->d_keys_out, (uint32_t)nwin, whead, s);
-    if ((rc = flag_scan(c, whead, hw, nwin))) return rc;
-  }
-  launch_window_offsets(c->d_keys_out, whead, (uint32_t)nwin, nwp, cam.d_wseg_off, s);
-  // C with its window part summed per segment, and the front messages
-  launch_pair_finish(cam.d_inc + nrec_f, c->d_keys_out, cam.d_win_idx, (uint32_t)nwin, nwp, acc_w, acc_f, acc_r, np,
-                     cam.d_pair_c, cam.d_pair_sf, s);
-  // 7. window segment head bitmask and per-tile head counts
+  // ... their layout (first positions, head bitmask, per-tile head counts), C
+  // and the front messages
   const size_t nwords_w = nwin / 64 + 1, ntiles_w = nwin / kTile + 1;
   if ((rc = dalloc(c, &cam.d_heads, nwords_w)) || (rc = dalloc(c, &cam.d_tile_h0, ntiles_w))) return rc;
-  launch_pack_flags(whead, hw, (uint32_t)nwin, cam.d_heads, cam.d_tile_h0, s);
+  launch_window_layout(cam.d_inc + nrec_f, c->d_keys_out, cam.d_win_idx, (uint32_t)nwin, nwp, cam.d_wseg_off,
+                       cam.d_heads, cam.d_tile_h0, acc_f, acc_w, acc_r, cam.d_pair_c, cam.d_pair_sf, s);
+  launch_pair_finish(acc_w, acc_f, acc_r, cam.d_wseg_off, np, nwp, cam.d_pair_c, cam.d_pair_sf, s);
   if (keep_msgs)
     launch_gather_pairs(cam.d_pair_vox, c->d_A, np, cam.d_M, s);
   else
@@ -891,7 +881,7 @@ int prepare(mrf_ctx* c) {
       dfree(&cam.d_dyn);
       if ((rc = dalloc(c, &cam.d_dyn, std::max<uint32_t>(nrest, 1)))) return rc;
       if ((rc = ensure_sort(c, std::max<size_t>(cam.nchunks, 1), 1))) return rc;
-      uint32_t* crow = c->d_x0;  // sort scratch of at least nchunks words: rows per chunk
+      uint32_t* crow = c->d_keys_in;  // sort scratch of at least nchunks words: rows per chunk
       launch_zero_words(c->d_total + 2, 8, c->stream);
       launch_zero_words(c->d_total + 8, 16, c->stream);
       if (nrest) {
@@ -1432,7 +1422,6 @@ void mrf_destroy(mrf_ctx* c) {
   dfree(&c->d_Spair);
   dfree(&c->d_pf_v); dfree(&c->d_pl_v); dfree(&c->d_mid);
   dfree(&c->d_keys_in); dfree(&c->d_keys_out); dfree(&c->d_vals_in);
-  dfree(&c->d_x0); dfree(&c->d_x1);
   dfree(&c->d_vflag); dfree(&c->d_acc); dfree(&c->d_sell0);
   dfree(&c->d_eval); dfree(&c->d_eval_part); dfree(&c->d_eval_counts);
   dfree(&c->d_wpass); dfree(&c->d_wmsum); dfree(&c->d_wmmax); dfree(&c->d_wdelta);

@@ -195,7 +195,7 @@ __device__ __forceinline__ void wave_seg_sum_u(uint32_t& x, uint32_t& x2, uint32
 // window.  Front runs go to the front sum acc_f and their parts below 2^-24
 // to acc_r; a window row only has its records rewritten: the window part of
 // C is summed after the window sort, where each pair's records are already
-// contiguous (k_window_lengths).  C is the window part plus acc_f plus acc_r.
+// contiguous (k_window_layout).  C is the window part plus acc_f plus acc_r.
 // PACKED (fewer than 2^26 - 1 pairs): the sort moves one word per lane, the
 // pair and the lane it came from (pair 2^6 + lane, unique), and each lane then
 // fetches its lengths from that lane; else (pair, q, r) move together.
@@ -289,91 +289,140 @@ __global__ void __launch_bounds__(256) k_pair_lengths(uint2* __restrict__ rec, u
   }
 }
 
-// The window part of C of every window pair, from the sorted window records
-// (position m holds pair keys[m], record win_idx[m] of the window region): a
-// wave takes 64 consecutive positions, computes the same exact fixed-point
-// parts as k_pair_lengths, sums each run of equal pairs (segmented scan; the
-// runs are already contiguous) and adds it with one exact add per run into
-// acc_w (2^-24 units) and acc_r (below): one add per segment and wave it
-// touches, instead of one per run of every window row.
-__global__ __launch_bounds__(256) void k_window_lengths(const uint2* __restrict__ recw,
-                                                        const uint32_t* __restrict__ keys,
-                                                        const uint32_t* __restrict__ win_idx, uint32_t nwin,
-                                                        uint32_t* __restrict__ acc_w, uint32_t* __restrict__ acc_r) {
-  const int lane = threadIdx.x & 63;
-  const uint32_t m0 = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64u;
-  if (m0 >= nwin) return;  // uniform per wavefront
-  const uint32_t m = m0 + (uint32_t)lane;
-  const bool valid = m < nwin;
-  uint32_t key = 0xFFFFFFFFu, q = 0, r = 0;
-  if (valid) {
-    key = keys[m];
-    const double x = (double)__uint_as_float(recw[win_idx[m]].y) * kFixLen;
-    q = (uint32_t)x;
-    r = (uint32_t)((x - (double)q) * kFixLen);
-  }
-  const uint32_t prev = (uint32_t)__shfl_up((int)key, 1, 64);
-  const uint32_t next = (uint32_t)__shfl_down((int)key, 1, 64);
-  wave_seg_sum_u(q, r, lane == 0 || prev != key ? 1u : 0u);
-  if ((lane == 63 || next != key) && key != 0xFFFFFFFFu) {
-    uint32_t* pw = acc_w + 2 * (size_t)key;
-    const uint32_t o = atomicAdd(pw, q);
-    if (o + q < o) atomicAdd(pw + 1, 1u);
-    if (r) {
-      uint32_t* pr = acc_r + 2 * (size_t)key;
-      const uint32_t orr = atomicAdd(pr, r);
-      if (orr + r < orr) atomicAdd(pr + 1, 1u);
-    }
-  }
-}
-
-// C in FP32 with the gate of the exact sum (C > 0.1f, gvdbkernels.cu:408):
-// where rounding to float would move C onto kCumLenMin from above, C takes
-// the next float up, so that the float gate falls as on the exact sum
-__global__ void k_pair_finish(const uint32_t* __restrict__ acc_w, const uint32_t* __restrict__ acc_f,
-                              const uint32_t* __restrict__ acc_r, uint32_t np, uint32_t nwp,
-                              float* __restrict__ pair_c, float* __restrict__ pair_sf) {
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  // integers below 2^53: the doubles and their sum are exact; a front-only
-  // pair has no window part
-  const double w = p < nwp ? (double)acc_w[2 * p + 1] * 4294967296.0 + (double)acc_w[2 * p] : 0.0;
-  const double cr = (double)acc_r[2 * p + 1] * 4294967296.0 + (double)acc_r[2 * p];
-  const double f = (double)acc_f[2 * p + 1] * 4294967296.0 + (double)acc_f[2 * p];
-  const double cd = (w + f) / kFixLen + cr / (kFixLen * kFixLen);
+// C in FP32 with the gate of the exact sum (C > 0.1f, gvdbkernels.cu:408) from
+// the exact fixed-point sums of a pair: w, f in units of 2^-24 (window, front
+// records), r the parts below in units of 2^-48.  Where rounding to float
+// would move C onto kCumLenMin from above, C takes the next float up, so that
+// the float gate falls as on the exact sum.  The integers are below 2^53: the
+// doubles and their sum are exact.
+__device__ __forceinline__ float pair_length(uint64_t w, uint64_t f, uint64_t r) {
+  const double cd = ((double)w + (double)f) / kFixLen + (double)r / (kFixLen * kFixLen);
   float cf = (float)cd;
   if (cd > (double)kCumLenGate) {
     if (!(cf > kCumLenMin)) cf = __uint_as_float(__float_as_uint(kCumLenMin) + 1u);
   } else if (cf > kCumLenMin) {
     cf = kCumLenMin;
   }
-  pair_c[p] = cf;
-  pair_sf[p] = (float)((double)kFEps * (f / kFixLen));
+  return cf;
+}
+// F_EPS x the chord length of the front records
+__device__ __forceinline__ float front_message(uint64_t f) { return (float)((double)kFEps * ((double)f / kFixLen)); }
+
+// Segment layout of the sorted window records (position m holds pair keys[m],
+// record win_idx[m] of the window region) and C of the window pairs, a wave
+// per tile of kTile positions.  Every window pair has live window records, so
+// the sorted keys step through 0, 1, 2, ...: the key of a head is the number
+// of heads before it, and the first position of a pair (wseg_off), the head
+// bitmask and the heads before a tile (tile_h0) need no scan.  The lengths
+// become the exact fixed-point parts of k_reslice; runs of equal pairs are
+// summed by a segmented scan per row of 64, a row's last run is carried into
+// the next row.  A pair whose records all lie in this tile is finished here;
+// of the others, the part in this tile is added to acc_w (units of 2^-24,
+// zeroed before) and acc_r, and k_pair_finish ends them.
+// Bound by its loads, so all of them are in flight before the first is used
+// (keys and indices, then the gathered records with the pairs' front sums)
+// and every store comes after the last.  640x480 at 1 cm, 30 M positions: 313
+// us and 62 us for k_pair_finish; heads, scan, offsets and bits as passes of
+// their own with atomic length sums took 281 + 292 us and 79 us.
+__global__ __launch_bounds__(256) void k_window_layout(const uint2* __restrict__ recw,
+                                                       const uint32_t* __restrict__ keys,
+                                                       const uint32_t* __restrict__ win_idx, uint32_t nwin,
+                                                       uint32_t nwp, uint32_t* __restrict__ wseg_off,
+                                                       uint64_t* __restrict__ bits, uint32_t* __restrict__ tile_h0,
+                                                       const uint64_t* __restrict__ acc_f,
+                                                       unsigned long long* acc_w, unsigned long long* acc_r,
+                                                       float* __restrict__ pair_c, float* __restrict__ pair_sf) {
+  constexpr int kRows = kTile / 64;
+  const int lane = threadIdx.x & 63;
+  const uint32_t tile = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (tile == 0 && lane == 0) wseg_off[nwp] = nwin;
+  if ((uint64_t)tile * kTile >= nwin) return;  // uniform per wavefront
+  const uint32_t m0 = tile * kTile;
+  uint32_t key[kRows], len[kRows], next[kRows];
+#pragma unroll
+  for (int j = 0; j < kRows; ++j) {
+    const uint32_t m = m0 + 64u * j + lane;
+    key[j] = m < nwin ? keys[m] : 0xFFFFFFFFu;
+    len[j] = m < nwin ? win_idx[m] : 0u;
+  }
+  // the keys on either side of the tile (no pair: none)
+  const uint32_t left = m0 ? keys[m0 - 1] : 0xFFFFFFFFu;
+  const uint32_t right = m0 + kTile < nwin ? keys[m0 + kTile] : 0xFFFFFFFFu;
+#pragma unroll
+  for (int j = 0; j < kRows; ++j) {
+    const uint32_t after = j + 1 < kRows ? (uint32_t)__builtin_amdgcn_readfirstlane((int)key[j + 1 < kRows ? j + 1 : j])
+                                         : right;
+    const uint32_t down = (uint32_t)__shfl_down((int)key[j], 1, 64);
+    next[j] = lane == 63 ? after : down;
+  }
+  // a run's last lane, of a pair that lies in the tile: f its front sum, r the parts below
+  uint64_t f[kRows], r[kRows];
+#pragma unroll
+  for (int j = 0; j < kRows; ++j) {
+    len[j] = key[j] != 0xFFFFFFFFu ? recw[len[j]].y : 0u;
+    const bool done = key[j] != 0xFFFFFFFFu && next[j] != key[j] && key[j] != left;
+    f[j] = done ? acc_f[key[j]] : 0u;
+    r[j] = done ? acc_r[key[j]] : 0u;
+  }
+  uint64_t w[kRows], hb[kRows];
+  uint32_t before = left;             // the key before the row
+  uint64_t carry_w = 0, carry_r = 0;  // the run that goes on from the row before
+#pragma unroll
+  for (int j = 0; j < kRows; ++j) {
+    const uint32_t k = key[j];
+    const uint32_t up = (uint32_t)__shfl_up((int)k, 1, 64), prev = lane == 0 ? before : up;
+    hb[j] = __ballot(k != 0xFFFFFFFFu && prev != k);
+    // l 2^24 is exact in double; ql its integer part (< 2^25), rl the rest in
+    // units of 2^-48 (< 2^24)
+    const double x = (double)__uint_as_float(len[j]) * kFixLen;
+    uint32_t ql = (uint32_t)x;
+    uint32_t rl = (uint32_t)((x - (double)ql) * kFixLen);
+    wave_seg_sum_u(ql, rl, lane == 0 || prev != k ? 1u : 0u);
+    const bool goes_on = (hb[j] & (~0ull >> (63 - lane))) == 0;  // still in the run from before the row
+    w[j] = ql + (goes_on ? carry_w : 0u);
+    const uint64_t rj = rl + (goes_on ? carry_r : 0u);
+    r[j] += rj;
+    before = (uint32_t)__builtin_amdgcn_readlane((int)k, 63);
+    const bool carries = before == (uint32_t)__builtin_amdgcn_readlane((int)next[j], 63);
+    const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)w[j], 63),
+                   w1 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(w[j] >> 32), 63),
+                   r0 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)rj, 63),
+                   r1 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(rj >> 32), 63);
+    carry_w = carries ? (uint64_t)w0 | (uint64_t)w1 << 32 : 0u;
+    carry_r = carries ? (uint64_t)r0 | (uint64_t)r1 << 32 : 0u;
+  }
+  if (lane == 0) tile_h0[tile] = hb[0] & 1u ? key[0] : key[0] + 1u;
+#pragma unroll
+  for (int j = 0; j < kRows; ++j) {
+    const uint32_t m = m0 + 64u * j + lane, k = key[j];
+    if (lane == 0 && m < nwin) bits[m >> 6] = hb[j];
+    if ((hb[j] >> lane) & 1u) wseg_off[k] = m;
+    if (k == 0xFFFFFFFFu) continue;
+    if (next[j] != k && k != left) {
+      pair_c[k] = pair_length(w[j], f[j], r[j]);
+      pair_sf[k] = front_message(f[j]);
+    } else if (next[j] != k || (j + 1 == kRows && lane == 63)) {  // from or into another tile
+      atomicAdd(acc_w + k, (unsigned long long)w[j]);
+      if (r[j]) atomicAdd(acc_r + k, (unsigned long long)r[j]);
+    }
+  }
 }
 
-__global__ void k_window_heads(const uint32_t* __restrict__ keys, uint32_t nwin, uint32_t* __restrict__ whead) {
-  const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= nwin) return;
-  whead[m] = (m == 0 || keys[m - 1] != keys[m]) ? 1u : 0u;
-}
-
-__global__ void k_window_offsets(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ whead, uint32_t nwin,
-                                 uint32_t nwp, uint32_t* __restrict__ wseg_off) {
-  const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < nwin && whead[m]) wseg_off[keys[m]] = m;
-  if (m == 0) wseg_off[nwp] = nwin;
-}
-
-__global__ void k_pack_flags(const uint32_t* __restrict__ flags, uint32_t n, uint64_t* __restrict__ bits) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;  // blockDim is a multiple of 64
-  const bool h = j < n && flags[j] != 0u;
-  const unsigned long long word = __ballot(h);
-  if ((threadIdx.x & 63) == 0 && j < n) bits[j >> 6] = word;
-}
-
-__global__ void k_tile_h0(const uint32_t* __restrict__ fscan, uint32_t n, uint32_t* __restrict__ tile_h0) {
-  const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w * kTile < n) tile_h0[w] = fscan[w * kTile];
+// C and the front messages of the pairs that k_window_layout left: the
+// front-only pairs and the window pairs whose records cross a tile's end
+__global__ void k_pair_finish(const uint64_t* __restrict__ acc_w, const uint64_t* __restrict__ acc_f,
+                              const uint64_t* __restrict__ acc_r, const uint32_t* __restrict__ wseg_off, uint32_t np,
+                              uint32_t nwp, float* __restrict__ pair_c, float* __restrict__ pair_sf) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= np) return;
+  uint64_t w = 0;
+  if (p < nwp) {
+    if (wseg_off[p] / kTile == (wseg_off[p + 1] - 1u) / kTile) return;
+    w = acc_w[p];
+  }
+  const uint64_t f = acc_f[p];
+  pair_c[p] = pair_length(w, f, acc_r[p]);
+  pair_sf[p] = front_message(f);
 }
 
 // record -> voxel (for export)
@@ -428,16 +477,20 @@ void launch_pair_lengths(uint2* rec, uint64_t nrec, uint64_t base_w, const uint3
                        acc_f, acc_r, wkeys, wvals, sentinel);
 }
 
-void launch_pair_finish(const uint2* recw, const uint32_t* keys, const uint32_t* win_idx, uint32_t nwin,
-                        uint32_t nwp, uint32_t* acc_w, const uint32_t* acc_f, uint32_t* acc_r, uint32_t np,
-                        float* pair_c, float* pair_sf, hipStream_t s) {
-  if (np == 0) return;
+void launch_window_layout(const uint2* recw, const uint32_t* keys, const uint32_t* win_idx, uint32_t nwin,
+                          uint32_t nwp, uint32_t* wseg_off, uint64_t* bits, uint32_t* tile_h0, const uint64_t* acc_f,
+                          uint64_t* acc_w, uint64_t* acc_r, float* pair_c, float* pair_sf, hipStream_t s) {
   launch_zero_words(acc_w, (size_t)nwp * 8, s);
-  if (nwin)
-    hipLaunchKernelGGL(k_window_lengths, dim3(blocks(nwin, 256)), dim3(256), 0, s, recw, keys, win_idx, nwin, acc_w,
-                       acc_r);
-  hipLaunchKernelGGL(k_pair_finish, dim3(blocks(np, 256)), dim3(256), 0, s, acc_w, acc_f, acc_r, np, nwp, pair_c,
-                     pair_sf);
+  hipLaunchKernelGGL(k_window_layout, dim3(blocks(nwin ? nwin : 1, 4 * kTile)), dim3(256), 0, s, recw, keys, win_idx,
+                     nwin, nwp, wseg_off, bits, tile_h0, acc_f, reinterpret_cast<unsigned long long*>(acc_w),
+                     reinterpret_cast<unsigned long long*>(acc_r), pair_c, pair_sf);
+}
+
+void launch_pair_finish(const uint64_t* acc_w, const uint64_t* acc_f, const uint64_t* acc_r, const uint32_t* wseg_off,
+                        uint32_t np, uint32_t nwp, float* pair_c, float* pair_sf, hipStream_t s) {
+  if (np == 0) return;
+  hipLaunchKernelGGL(k_pair_finish, dim3(blocks(np, 256)), dim3(256), 0, s, acc_w, acc_f, acc_r, wseg_off, np, nwp,
+                     pair_c, pair_sf);
 }
 
 hipError_t sort_window(uint32_t nwr, int bits, uint32_t* keys_in, uint32_t* keys_out, uint32_t* vals_in,
@@ -445,25 +498,6 @@ hipError_t sort_window(uint32_t nwr, int bits, uint32_t* keys_in, uint32_t* keys
   if (nwr == 0) return hipSuccess;
   size_t tb = temp_bytes;
   return hipcub::DeviceRadixSort::SortPairs(temp, tb, keys_in, keys_out, vals_in, vals_out, (int)nwr, 0, bits, s);
-}
-
-void launch_window_heads(const uint32_t* keys, uint32_t nwin, uint32_t* whead, hipStream_t s) {
-  if (nwin == 0) return;
-  hipLaunchKernelGGL(k_window_heads, dim3(blocks(nwin, 256)), dim3(256), 0, s, keys, nwin, whead);
-}
-
-void launch_window_offsets(const uint32_t* keys, const uint32_t* whead, uint32_t nwin, uint32_t nwp,
-                           uint32_t* wseg_off, hipStream_t s) {
-  hipLaunchKernelGGL(k_window_offsets, dim3(blocks(nwin ? nwin : 1, 256)), dim3(256), 0, s, keys, whead, nwin, nwp,
-                     wseg_off);
-}
-
-void launch_pack_flags(const uint32_t* flags, const uint32_t* fscan, uint32_t n, uint64_t* bits, uint32_t* tile_h0,
-                       hipStream_t s) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_pack_flags, dim3(blocks(n, 256)), dim3(256), 0, s, flags, n, bits);
-  const uint32_t ntiles = (n + kTile - 1) / kTile;
-  hipLaunchKernelGGL(k_tile_h0, dim3(blocks(ntiles, 256)), dim3(256), 0, s, fscan, n, tile_h0);
 }
 
 void launch_export_vox(const uint2* rec, uint32_t n, const uint32_t* pair_vox, uint2* out, hipStream_t s) {

@@ -96,26 +96,24 @@ void launch_pair_lengths(uint2* rec, uint64_t nrec, uint64_t base_w, const uint3
                          uint32_t* acc_r, uint32_t np, uint32_t* wkeys, uint32_t* wvals, uint32_t sentinel,
                          hipStream_t s);
 // after the window sort (sorted pair keys and win_idx of the nwin live
-// window records): the window part of every window pair (acc_w; the parts
-// below 2^-24 into acc_r), then per pair C (summed chord length, exact, FP32
-// with the exact sum's gate) and F_EPS x the chord length of its front
-// records
-void launch_pair_finish(const uint2* recw, const uint32_t* keys, const uint32_t* win_idx, uint32_t nwin,
-                        uint32_t nwp, uint32_t* acc_w, const uint32_t* acc_f, uint32_t* acc_r, uint32_t np,
-                        float* pair_c, float* pair_sf, hipStream_t s);
+// window records), the segment layout: wseg_off[pair] = first window position
+// of the pair, wseg_off[nwp] = nwin; the bitmask of the segment heads; per
+// kTile tile the heads before it.  And per pair C (summed chord length, exact,
+// FP32 with the exact sum's gate) and F_EPS x the chord length of its front
+// records: launch_window_layout finishes the window pairs within a tile and
+// leaves the sums of the others in acc_w and acc_r, launch_pair_finish ends
+// all the others
+void launch_window_layout(const uint2* recw, const uint32_t* keys, const uint32_t* win_idx, uint32_t nwin,
+                          uint32_t nwp, uint32_t* wseg_off, uint64_t* bits, uint32_t* tile_h0, const uint64_t* acc_f,
+                          uint64_t* acc_w, uint64_t* acc_r, float* pair_c, float* pair_sf, hipStream_t s);
+void launch_pair_finish(const uint64_t* acc_w, const uint64_t* acc_f, const uint64_t* acc_r, const uint32_t* wseg_off,
+                        uint32_t np, uint32_t nwp, float* pair_c, float* pair_sf, hipStream_t s);
 size_t window_sort_temp_bytes(uint32_t n, int bits);
 // window region records stably sorted by pair (gap / padding records, with
 // the sentinel key, last): keys_out = pairs, vals_out = record index in the
 // region
 hipError_t sort_window(uint32_t nwr, int bits, uint32_t* keys_in, uint32_t* keys_out, uint32_t* vals_in,
                        uint32_t* vals_out, void* temp, size_t temp_bytes, hipStream_t s);
-void launch_window_heads(const uint32_t* keys, uint32_t nwin, uint32_t* whead, hipStream_t s);
-// wseg_off[pair] = first window position of the pair, wseg_off[nwp] = nwin
-void launch_window_offsets(const uint32_t* keys, const uint32_t* whead, uint32_t nwin, uint32_t nwp,
-                           uint32_t* wseg_off, hipStream_t s);
-// flag bitmask (bit j = flags[j] != 0) and, per kTile tile, fscan at its start
-void launch_pack_flags(const uint32_t* flags, const uint32_t* fscan, uint32_t n, uint64_t* bits, uint32_t* tile_h0,
-                       hipStream_t s);
 // records with their voxel ids restored (for export)
 void launch_export_vox(const uint2* rec, uint32_t n, const uint32_t* pair_vox, uint2* out, hipStream_t s);
 

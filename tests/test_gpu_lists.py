@@ -35,6 +35,7 @@ def _room(rows, cols, focal, near, far, vis, seed=5):
     (8, 8, 9.0, 0.05, 0.3),    # one tile, rays of window records only and short fronts
     (9, 17, 12.0, 0.1, 1.8),   # ragged tiles, rays of every length, beyond the grid
     (40, 24, 30.0, 1.6, 1.8),  # long fronts, several batches per slice
+    (48, 48, 400.0, 0.3, 0.4), # voxels met by every ray: segments over several 512-position tiles
 ])
 def test_lists_and_marginals_match_oracle(rows, cols, focal, near, far, vis):
     """Lists bit for bit; marginals after 2 iterations within the 1e-3 that
