@@ -117,7 +117,7 @@ struct mrf_ctx {
   size_t cap_sort = 0;
   uint32_t* d_vflag = nullptr;  // 4 pool-sized tables: touched, window-touched and their scans
   size_t cap_vflag = 0;
-  uint64_t* d_acc = nullptr;  // per pair three fixed-point chord-length sums
+  uint64_t* d_acc = nullptr;  // per pair up to four words of fixed-point chord-length sums
   size_t cap_acc = 0;
   uint2* d_sell0 = nullptr;
   size_t cap_sell0 = 0;
@@ -561,7 +561,7 @@ int ensure_acc(mrf_ctx* c, size_t np) {
   np += np / 4;
   dfree(&c->d_acc);
   c->cap_acc = 0;
-  int rc = dalloc(c, &c->d_acc, 3 * np);
+  int rc = dalloc(c, &c->d_acc, 4 * np);
   if (rc) return rc;
   c->cap_acc = np;
   return MRF_OK;
@@ -658,6 +658,8 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   if ((rc = ensure_sell0(c, std::max<uint64_t>(nrec0, 1))) || (rc = dalloc(c, &cam.d_front, npix)) ||
       (rc = dalloc(c, &cam.d_lanes, npix)))
     return rc;
+  uint32_t* ids = reinterpret_cast<uint32_t*>(c->d_sell0);  // staged voxels, then the chord lengths
+  uint32_t* lens = ids + c->cap_sell0;
   uint32_t* overflow = reinterpret_cast<uint32_t*>(c->d_total + 6);
   launch_zero_words(overflow, 8, s);
   // 2. the emission splits each ray into front and window (counts into
@@ -667,7 +669,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   // (with full-ray activation every brick on a ray's way is active; the
   // staged ids then hold the linear brick index, below 2^23 for the sentinel)
   const bool all_active = cam.d_walkn && c->nbricks < (1 << 23);
-  launch_emit(cg, c->g, cam.d_depth, c->d_sig, c->d_bia, c->d_slot, c->d_offs, c->d_has, c->d_sell0, cam.d_front,
+  launch_emit(cg, c->g, cam.d_depth, c->d_sig, c->d_bia, c->d_slot, c->d_offs, c->d_has, ids, c->cap_sell0, cam.d_front,
               cam.d_lanes, c->d_counts, c->d_rayidx, overflow, all_active, s);
   if ((rc = dalloc(c, &cam.d_len_f, ntiles)) || (rc = dalloc(c, &cam.d_len_w, ntiles)) ||
       (rc = dalloc(c, &cam.d_chunk_off, (size_t)ntiles + 1)))
@@ -693,8 +695,8 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   cam.base_w = nrec_f;
   cam.nslices = ntiles;
   if ((rc = dalloc(c, &cam.d_inc, nrec))) return rc;
-  // 3. the records into their regions; the voxels of live records (any) and
-  //    of live window records (wany), and the counts of both
+  // 3. the voxels of live records (any) and of live window records (wany),
+  //    and the counts of both
   const uint64_t nvox = (uint64_t)c->slot_lin.size() * kBrickVox;
   if ((rc = ensure_vflags(c, std::max<uint64_t>(nvox, 1)))) return rc;
   uint8_t* any = reinterpret_cast<uint8_t*>(c->d_vflag);  // byte flags
@@ -715,9 +717,9 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
     if ((rc = dalloc(c, &cam.d_bstart, wrows + 32)) || (rc = dalloc(c, &cam.d_tail, npix))) return rc;
     launch_zero_words(cam.d_bstart + wrows, 32 * sizeof(uint64_t), s);
   }
-  launch_reslice(cam.d_front, cam.d_lanes, ntiles, c->d_sell0, all_active ? c->d_slot : nullptr, c->d_offs, cam.d_len_f,
-                 c->d_has, cam.d_len_w, (uint32_t)nrec_f, cam.d_inc, any, wany, cam.d_bstart, cam.d_tail,
-                 (unsigned long long*)(c->d_total + 2), s);
+  const int32_t* brick_slot = all_active ? c->d_slot : nullptr;
+  launch_mark_voxels(cam.d_front, cam.d_lanes, ntiles, ids, brick_slot, cam.d_len_f, c->d_has, cam.d_len_w, any, wany,
+                     cam.d_bstart, cam.d_tail, (unsigned long long*)(c->d_total + 2), s);
   // one allocation for the partial sums, the static sums and the masks of
   // changing records (per chunk and lane each)
   const size_t nparts = (size_t)cam.nchunks * kSlice;
@@ -727,9 +729,8 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   cam.d_fstatic = cam.d_partial + nparts;
   cam.d_fdmask = reinterpret_cast<uint32_t*>(cam.d_partial + 2 * nparts);
   launch_chunk_desc(cam.d_chunk_off, cam.d_len_f, ntiles, cam.d_chunk_desc, s);
-  launch_front_span(cam.d_front, cam.d_lanes, ntiles * kSlice, cam.d_fspan, s);
   // 4. (camera, voxel) pairs: window pairs first, each group in voxel order.
-  //    One readback: [0..3] the reslice counters (live records, live window
+  //    One readback: [0..3] the counters (live records, live window
   //    records, records with gap records, rays with records), [4] the
   //    emission's overflow flag, [6] the pairs | the window pairs << 32
   launch_brick_flag_counts(any, wany, nbr, bcnt, s);
@@ -756,8 +757,9 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
       (rc = ensure_acc(c, std::max<uint32_t>(np, 1))))
     return rc;
   launch_pair_table(any, wany, boff, nbr, nwp, pid, cam.d_pair_vox, s);
-  // 5. per pair: the front parts of C; records point at their pairs from
-  //    here on.  The same pass writes the window sort's input
+  // 5. the records into their regions, pointing at their pairs from here on;
+  //    the same pass sums the front parts of C and writes the window sort's
+  //    input
   const int wbits = std::max(1, bit_length(nwp));
   if ((rc = ensure_sort(c, std::max<uint64_t>(nrec_w, 1), wbits))) return rc;
   // win_idx holds the sorted values of the whole window region; its first
@@ -765,10 +767,13 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   if ((rc = dalloc(c, &cam.d_wseg_off, (size_t)nwp + 1)) ||
       (rc = dalloc(c, &cam.d_win_idx, std::max<uint64_t>(nrec_w, 1))))
     return rc;
-  uint64_t* acc_w = c->d_acc;
-  uint64_t* acc_f = c->d_acc + (size_t)np;
-  uint64_t* acc_r = c->d_acc + 2 * (size_t)np;
-  launch_pair_lengths(cam.d_inc, nrec, nrec_f, pid, (uint32_t*)acc_f, (uint32_t*)acc_r, np, c->d_keys_in, c->d_vals_in, nwp, s);
+  uint64_t* acc = c->d_acc;
+  uint64_t* acc_hi = acc + np;
+  uint64_t* acc_w = acc_hi + np;
+  uint64_t* acc_r = acc_w + nwp;
+  launch_reslice(cam.d_front, cam.d_lanes, ntiles, ids, lens, brick_slot, pid, c->d_offs, cam.d_len_f, c->d_has,
+                 cam.d_len_w, (uint32_t)nrec_f, cam.d_inc, acc, acc_hi, np, c->d_keys_in, c->d_vals_in, nwp, s);
+  launch_front_span(cam.d_front, cam.d_lanes, ntiles * kSlice, cam.d_fspan, s);
   // 6. window segments: the window records stably sorted by pair
   HIPCHK(c, sort_window((uint32_t)nrec_w, wbits, c->d_keys_in, c->d_keys_out, c->d_vals_in, cam.d_win_idx,
                         c->d_sort_tmp, c->sort_tmp_bytes, s));
@@ -777,8 +782,8 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   const size_t nwords_w = nwin / 64 + 1, ntiles_w = nwin / kTile + 1;
   if ((rc = dalloc(c, &cam.d_heads, nwords_w)) || (rc = dalloc(c, &cam.d_tile_h0, ntiles_w))) return rc;
   launch_window_layout(cam.d_inc + nrec_f, c->d_keys_out, cam.d_win_idx, (uint32_t)nwin, nwp, cam.d_wseg_off,
-                       cam.d_heads, cam.d_tile_h0, acc_f, acc_w, acc_r, cam.d_pair_c, cam.d_pair_sf, s);
-  launch_pair_finish(acc_w, acc_f, acc_r, cam.d_wseg_off, np, nwp, cam.d_pair_c, cam.d_pair_sf, s);
+                       cam.d_heads, cam.d_tile_h0, acc, acc_hi, acc_w, acc_r, cam.d_pair_c, cam.d_pair_sf, s);
+  launch_pair_finish(acc, acc_hi, acc_w, acc_r, cam.d_wseg_off, np, nwp, cam.d_pair_c, cam.d_pair_sf, s);
   if (keep_msgs)
     launch_gather_pairs(cam.d_pair_vox, c->d_A, np, cam.d_M, s);
   else

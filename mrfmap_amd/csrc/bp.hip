@@ -149,15 +149,13 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 }
 
 // ---------------------------------------------------------------- list layout
-// Copy every ray's records into the front and window regions of the final
-// record buffer (sliced: lane l of slice t at region offset + k * 64 + l),
-// padding each lane to its slice's length with gap records.  Record k of the
-// 64 rays of a slice moves together: per row the voxel flags any[v] = 1
-// (every live record) and wany[v] = 1 (live window records) are set, skipping
-// a lane whose voxel equals that of the ray to its left or above in the pixel
-// tile (the flags say only whether), and counts[0] / counts[1] gain the row's
-// live / live window records; counts[2] gains the slice's records (gap
-// records included) and counts[3] its rays with records.
+// The voxels of every ray's staged records: per row (record k of the 64 rays
+// of a slice) the voxel flags any[v] = 1 (every live record) and wany[v] = 1
+// (live window records) are set, skipping a lane whose voxel equals that of
+// the ray to its left or above in the pixel tile (the flags say only
+// whether), and counts[0] / counts[1] gain the row's live / live window
+// records; counts[2] gains the slice's records (gap records included) and
+// counts[3] its rays with records.
 // SLOTS: the staged records hold (linear brick index) * 512 + voxel, and the
 // brick's slot is looked up here (neighbouring rays share their bricks).
 //
@@ -167,31 +165,31 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 // exist.  The 64 lanes' flags of a window row form one 64-bit word.
 // tail[lane]: when the first window record continues the brick of the last
 // front record, the number of front records since that brick's entry (at most
-// 22, the longest crossing of a brick), else 0.  Both look one record back,
-// at the staged copy.
+// 22, the longest crossing of a brick), else 0.  Both look one record back.
 //
 // A block of four waves is one slice, batches of kB rows going to its waves
 // in turn: a wave's batch is a chain of loads (record, slot) before its
 // stores, and one wave per slice leaves four waves per SIMD at 640x480 and
-// fewer than one below 160x120.  640x480 at 1 cm, 161 M records, 2.6 GB read
-// and written: 795 us; one wave per slice and the brick entries as a pass of
-// their own took 869 + 116 us (160x120 at 4 cm: 30 us against 38 + 54).
+// fewer than one below 160x120.  640x480 at 1 cm, 161 M voxels (0.65 GB): 392
+// us, mostly the flags' byte stores; 160x120 at 4 cm: 27 us (with the copy in
+// the same pass 30, on one wave per slice and with the brick entries as a pass
+// of their own 92).
 template <bool SLOTS>
-__global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, RayRec* __restrict__ lanes,
-                                                 const uint2* __restrict__ sell, const int32_t* __restrict__ slot,
-                                                 const uint32_t* __restrict__ off_f, const uint32_t* __restrict__ len_f,
-                                                 const uint32_t* __restrict__ off_w, const uint32_t* __restrict__ len_w,
-                                                 uint32_t base_w, uint2* __restrict__ inc, uint8_t* __restrict__ any,
-                                                 uint8_t* __restrict__ wany, uint64_t* __restrict__ bstart,
-                                                 uint8_t* __restrict__ tail, unsigned long long* __restrict__ counts) {
+__global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict__ front,
+                                                     const RayRec* __restrict__ lanes,
+                                                     const uint32_t* __restrict__ ids, const int32_t* __restrict__ slot,
+                                                     const uint32_t* __restrict__ len_f,
+                                                     const uint32_t* __restrict__ off_w,
+                                                     const uint32_t* __restrict__ len_w, uint8_t* __restrict__ any,
+                                                     uint8_t* __restrict__ wany, uint64_t* __restrict__ bstart,
+                                                     uint8_t* __restrict__ tail,
+                                                     unsigned long long* __restrict__ counts) {
   constexpr uint32_t kW = 4, kB = 8;
   __shared__ uint64_t wave_counts[kW][2];
   const uint32_t t = blockIdx.x, wave = threadIdx.x >> 6, l = threadIdx.x & 63u, ray = t * kSlice + l;
   const FrontRec f = front[ray];
   const uint32_t rnw = lanes[ray].nw, nr = f.nf + rnw;
-  const uint2* __restrict__ src = sell + f.off;
-  const uint32_t fo = off_f[t] + l, wo = base_w + off_w[t] + l;
-  const uint2 gap = make_uint2(kGapVox, 0u);
+  const uint32_t* __restrict__ src = ids + f.off;
   // a voxel this lane need not flag: the left or the upper ray has it too
   auto dup = [&](uint32_t v) {
     const uint32_t left = (uint32_t)__shfl_up((int)v, 1, 64), up = (uint32_t)__shfl_up((int)v, 8, 64);
@@ -199,52 +197,43 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
   };
   // a batch's loads are in flight together (the bounds lf, lw are uniform per
   // wavefront, so every lane takes part in the shuffles)
-  auto pool_ids = [&](uint2(&e)[kB]) {
+  auto pool_ids = [&](uint32_t(&e)[kB]) {
     if constexpr (SLOTS) {
       int32_t sl[kB];
 #pragma unroll
-      for (uint32_t u = 0; u < kB; ++u) sl[u] = slot[e[u].x != kGapVox ? e[u].x >> kBrickLog * 3 : 0u];
+      for (uint32_t u = 0; u < kB; ++u) sl[u] = slot[e[u] != kGapVox ? e[u] >> kBrickLog * 3 : 0u];
 #pragma unroll
       for (uint32_t u = 0; u < kB; ++u)
-        if (e[u].x != kGapVox) e[u].x = (uint32_t)sl[u] * kBrickVox + (e[u].x & (kBrickVox - 1u));
+        if (e[u] != kGapVox) e[u] = (uint32_t)sl[u] * kBrickVox + (e[u] & (kBrickVox - 1u));
     }
   };
   uint64_t nl = 0, nw = 0;
   const uint32_t lf = len_f[t], lw = len_w[t];
   for (uint32_t k0 = wave * kB; k0 < lf; k0 += kW * kB) {
-    uint2 e[kB];
+    uint32_t e[kB];
 #pragma unroll
-    for (uint32_t u = 0; u < kB; ++u) {
-      e[u] = gap;
-      if (k0 + u < f.nf) e[u] = src[(size_t)(k0 + u) * kSlice];
-    }
+    for (uint32_t u = 0; u < kB; ++u) e[u] = k0 + u < f.nf ? src[(size_t)(k0 + u) * kSlice] : kGapVox;
     pool_ids(e);
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
-      if (k0 + u < lf) {
-        inc[fo + (size_t)(k0 + u) * kSlice] = e[u];
-        const bool live = e[u].x != kGapVox;
-        nl += (uint64_t)__popcll(__ballot(live));
-        const bool d = dup(e[u].x);
-        if (live && !d) any[e[u].x] = 1;
-      }
+      const bool live = e[u] != kGapVox;
+      nl += (uint64_t)__popcll(__ballot(live));
+      const bool d = dup(e[u]);
+      if (live && !d) any[e[u]] = 1;
     }
   }
-  const uint2* __restrict__ srcw = src + (size_t)f.nf * kSlice;
+  const uint32_t* __restrict__ srcw = src + (size_t)f.nf * kSlice;
   for (uint32_t k0 = wave * kB; k0 < lw; k0 += kW * kB) {
-    uint2 e[kB];
+    uint32_t e[kB];
     uint32_t prev = kGapVox;  // the ray's record before the batch
-    if (bstart && f.nf + k0 > 0 && k0 <= rnw) prev = src[(size_t)(f.nf + k0 - 1) * kSlice].x;
+    if (bstart && f.nf + k0 > 0 && k0 <= rnw) prev = src[(size_t)(f.nf + k0 - 1) * kSlice];
 #pragma unroll
-    for (uint32_t u = 0; u < kB; ++u) {
-      e[u] = gap;
-      if (k0 + u < rnw) e[u] = srcw[(size_t)(k0 + u) * kSlice];
-    }
+    for (uint32_t u = 0; u < kB; ++u) e[u] = k0 + u < rnw ? srcw[(size_t)(k0 + u) * kSlice] : kGapVox;
     if (bstart) {
       uint64_t mine = 0;  // lane u: the word of row k0 + u
 #pragma unroll
       for (uint32_t u = 0; u < kB; ++u) {
-        const uint32_t cur = e[u].x;
+        const uint32_t cur = e[u];
         const uint64_t m =
             __ballot(cur != kGapVox && (prev == kGapVox || (prev >> kBrickLog * 3) != (cur >> kBrickLog * 3)));
         if (l == u) mine = m;
@@ -255,24 +244,21 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
     pool_ids(e);
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
-      if (k0 + u < lw) {
-        inc[wo + (size_t)(k0 + u) * kSlice] = e[u];
-        const bool live = e[u].x != kGapVox;
-        const uint64_t n = (uint64_t)__popcll(__ballot(live));
-        nl += n;
-        nw += n;
-        const bool d = dup(e[u].x);
-        if (live && !d) {
-          any[e[u].x] = 1;
-          wany[e[u].x] = 1;
-        }
+      const bool live = e[u] != kGapVox;
+      const uint64_t n = (uint64_t)__popcll(__ballot(live));
+      nl += n;
+      nw += n;
+      const bool d = dup(e[u]);
+      if (live && !d) {
+        any[e[u]] = 1;
+        wany[e[u]] = 1;
       }
     }
   }
   if (tail && wave == kW - 1) {  // the wave with the fewest batches
     uint32_t tl = 0;
     if (f.nf && rnw) {
-      const uint32_t w0 = srcw[0].x, last = src[(size_t)(f.nf - 1) * kSlice].x;
+      const uint32_t w0 = srcw[0], last = src[(size_t)(f.nf - 1) * kSlice];
       auto same = [&](uint32_t v) { return v != kGapVox && (v >> kBrickLog * 3) == (w0 >> kBrickLog * 3); };
       if (w0 != kGapVox && same(last)) {
         bool more = true;
@@ -280,7 +266,7 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
           uint32_t pv[kB];
 #pragma unroll
           for (uint32_t u = 0; u < kB; ++u)
-            pv[u] = tl + u < f.nf ? src[(size_t)(f.nf - 1 - tl - u) * kSlice].x : kGapVox;
+            pv[u] = tl + u < f.nf ? src[(size_t)(f.nf - 1 - tl - u) * kSlice] : kGapVox;
 #pragma unroll
           for (uint32_t u = 0; u < kB; ++u) {
             more = more && same(pv[u]);
@@ -295,10 +281,8 @@ __global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, R
     wave_counts[wave][0] = nl;
     wave_counts[wave][1] = nw;
   }
-  __syncthreads();  // every wave has read the slice's descriptions as well
+  __syncthreads();
   if (wave != 0) return;
-  front[ray].off = fo;
-  lanes[ray].off_w = wo;
   // the slice's records (gap records included) and its rays with any
   const uint64_t nray = (uint64_t)__popcll(__ballot(nr != 0u));
   uint32_t nrec = nr;
@@ -1380,14 +1364,14 @@ void launch_epilogue(const CamPass& a, hipStream_t s, int part) {
                      a.npairs, a.wseg_off, a.S, a.pl_v, a.pf_v, a.mid, out_scale, a.B, a.M, a.upd, a.all_pairs);
 }
 
-void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t nslices, const uint2* sell, const int32_t* slot,
-                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
-                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail,
-                    unsigned long long* counts, hipStream_t s) {
+void launch_mark_voxels(const FrontRec* front, const RayRec* lanes, uint32_t nslices, const uint32_t* ids,
+                        const int32_t* slot, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
+                        uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail, unsigned long long* counts,
+                        hipStream_t s) {
   if (nslices == 0) return;
-  auto* k = slot ? k_reslice<true> : k_reslice<false>;
-  hipLaunchKernelGGL(k, dim3(nslices), dim3(256), 0, s, front, lanes, sell, slot, off_f, len_f, off_w, len_w, base_w, inc,
-                     any, wany, bstart, tail, counts);
+  auto* k = slot ? k_mark_voxels<true> : k_mark_voxels<false>;
+  hipLaunchKernelGGL(k, dim3(nslices), dim3(256), 0, s, front, lanes, ids, slot, len_f, off_w, len_w, any, wany, bstart,
+                     tail, counts);
 }
 
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s) {

@@ -12,20 +12,18 @@
 // accumulates with float atomics in every camera pass,
 // src/cuda/gvdbkernels.cu:519-571, 1276-1302) and the chord length of its
 // front records (whose messages are the constant F_EPS * l) are summed in
-// 2^-24 fixed point as 64-bit values kept in two 32-bit words: a 32-bit
-// atomic add to the low word, plus one to the high word when it wraps.  The
-// sums are exact, so they do not depend on the order in which records
-// arrive.  The part of each length below 2^-24 is summed the same way in
-// units of 2^-48, so C is exact for every chord of at least 2^-25 and the
-// epilogue gate C > 0.1f (gvdbkernels.cu:408) falls as it does on the exact
-// sum, however close to 0.1f C lies.
+// fixed point, each length as q 2^-24 + r 2^-48, both sums exact whatever
+// their size (the carries of the 32-bit words are kept), so they do not
+// depend on the order in which records arrive.  C is exact for every chord of
+// at least 2^-25, and the epilogue gate C > 0.1f (gvdbkernels.cu:408) falls as
+// it does on the exact sum, however close to 0.1f C lies.
 //
 // Window segments.  The window records are stably radix-sorted by pair, so
 // each pair's records stay in record order; the BP iteration sums each
 // segment in that order, gathered through win_idx (no atomics,
-// bit-reproducible).  The pass that sums the front part of C also rewrites
-// every live record to hold its pair instead of its voxel and writes the
-// sort's input.
+// bit-reproducible).  The pass that copies the records into their final
+// regions puts each live record's pair in place of its voxel, sums the front
+// part of C and writes the sort's input.
 #include <hipcub/hipcub.hpp>
 
 #include "mrf_kernels.h"
@@ -34,7 +32,7 @@ namespace mrf {
 
 namespace {
 
-constexpr double kFixLen = 16777216.0;  // 2^24: chord lengths (< 2) in fixed point, a 64-record sum < 2^31
+constexpr double kFixLen = 16777216.0;  // 2^24: chord lengths (< 1.74) in fixed point, a 64-record sum < 2^31
 
 // Pair numbering by brick (one wavefront per brick of the pool, 8 voxels
 // per lane, the byte flags read 8 at a time): a voxel's rank among the
@@ -100,64 +98,6 @@ __global__ __launch_bounds__(256) void k_pair_table(uint8_t* __restrict__ any, u
   if (w) *Wf = 0;
 }
 
-// value of lane ^ J; J < 32 stays inside the 32-lane half (ds_swizzle, bitmask mode)
-template <int J>
-__device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
-  if constexpr (J < 32)
-    return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (J << 10) | 0x1F);
-  else
-    return (uint32_t)__shfl_xor((int)v, J, 64);
-}
-
-// one bitonic step: lanes l and l ^ J order (key, val) ascending inside
-// blocks of K lanes whose index bit K is 0, descending otherwise
-template <int K, int J>
-__device__ __forceinline__ void bitonic_step(int lane, uint32_t& key, uint32_t& val, uint32_t& val2) {
-  const uint32_t ok = xor_lane<J>(key), ov = xor_lane<J>(val), ov2 = xor_lane<J>(val2);
-  const bool up = (lane & K) == 0;
-  const bool lower = (lane & J) == 0;
-  const bool take = (lower == up) ? (ok < key) : (ok > key);
-  key = take ? ok : key;
-  val = take ? ov : val;
-  val2 = take ? ov2 : val2;
-}
-
-template <int K, int J>
-__device__ __forceinline__ void bitonic_merge(int lane, uint32_t& key, uint32_t& val, uint32_t& val2) {
-  bitonic_step<K, J>(lane, key, val, val2);
-  if constexpr (J > 1) bitonic_merge<K, J / 2>(lane, key, val, val2);
-}
-
-// sorts key ascending over the K lanes, val and val2 travel with it
-template <int K>
-__device__ __forceinline__ void bitonic_sort(int lane, uint32_t& key, uint32_t& val, uint32_t& val2) {
-  if constexpr (K > 2) bitonic_sort<K / 2>(lane, key, val, val2);
-  bitonic_merge<K, K / 2>(lane, key, val, val2);
-}
-
-// Sort of one 32-bit value per lane over the 64 lanes, ascending; every
-// compare-exchange keeps the minimum in the lower lane.  Merging two sorted
-// halves of K lanes starts with the mirror partner l ^ (K - 1), then the
-// half-cleaners l ^ J, J = K/4 .. 1.
-template <int J>
-__device__ __forceinline__ void cx_min_low(int lane, int low_bit, uint32_t& v) {
-  const uint32_t o = xor_lane<J>(v);
-  v = (lane & low_bit) == 0 ? min(v, o) : max(v, o);
-}
-
-template <int K, int J>
-__device__ __forceinline__ void half_clean(int lane, uint32_t& v) {
-  cx_min_low<J>(lane, J, v);
-  if constexpr (J > 1) half_clean<K, J / 2>(lane, v);
-}
-
-template <int K>
-__device__ __forceinline__ void sort_u32(int lane, uint32_t& v) {
-  if constexpr (K > 2) sort_u32<K / 2>(lane, v);
-  cx_min_low<K - 1>(lane, K / 2, v);
-  if constexpr (K > 2) half_clean<K, K / 4>(lane, v);
-}
-
 template <int CTRL, int ROWS>
 __device__ __forceinline__ uint32_t dpp_u(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, true);
@@ -186,108 +126,172 @@ __device__ __forceinline__ void wave_seg_sum_u(uint32_t& x, uint32_t& x2, uint32
   seg_step_u<0x143, 0xC>(x, x2, f);
 }
 
-// A wave takes 64 consecutive records -- one step of the 64 rays of a pixel
-// tile, whose voxels repeat across neighbouring rays -- rewrites each live
-// record's voxel to its pair, sorts the 64 (pair, fixed-point length) by
-// pair across its lanes (bitonic network), sums each run of equal pairs
-// (segmented scan) and issues one atomic per run instead of one per record.
-// Regions are whole rows of 64 records, so a row is either all front or all
-// window.  Front runs go to the front sum acc_f and their parts below 2^-24
-// to acc_r; a window row only has its records rewritten: the window part of
-// C is summed after the window sort, where each pair's records are already
-// contiguous (k_window_layout).  C is the window part plus acc_f plus acc_r.
-// PACKED (fewer than 2^26 - 1 pairs): the sort moves one word per lane, the
-// pair and the lane it came from (pair 2^6 + lane, unique), and each lane then
-// fetches its lengths from that lane; else (pair, q, r) move together.
-// The same pass writes the window region's sort input: per window record j
-// (index base_w + j) key its pair (sentinel for a gap or padding record,
-// sorting last) and value j.
-template <bool PACKED>
-__global__ void __launch_bounds__(256) k_pair_lengths(uint2* __restrict__ rec, uint64_t nrec, uint64_t base_w,
-                                                      const uint32_t* __restrict__ pid,
-                                                      uint32_t* __restrict__ acc_f, uint32_t* __restrict__ acc_r,
-                                                      uint32_t* __restrict__ wkeys, uint32_t* __restrict__ wvals,
-                                                      uint32_t sentinel) {
-  // batches of kR rows per wave (nrec is a multiple of 64): the batch's
-  // records and then their pairs are loaded together, with no branches (a
-  // row past the end reads row 0 as gap records); the rows are sorted and
-  // summed; then the runs' exact adds {low word += q, high word += 1 if it
-  // wrapped} are issued, and their carries taken once the old values of all
-  // the batch's adds are back
-  constexpr int kR = 8;
-  const int lane = threadIdx.x & 63;
-  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-  const uint64_t nrows = nrec / 64;
-  for (uint64_t row0 = wave * kR; row0 < nrows; row0 += nwaves * kR) {
-    uint2 e[kR];
-    uint32_t key[kR], q[kR], r[kR];
+// Copy every ray's staged records into the front and window regions of the
+// final record buffer (sliced: lane l of slice t at region offset + k * 64 +
+// l), each live record with its pair instead of its voxel, padding each lane
+// to its slice's length with gap records; the window records' sort input (key
+// its pair, a sentinel that sorts last for a gap or padding record, value its
+// position in the region); and the front sums of every pair: acc holds
+// {sum of r (low word), sum of q (high word)} of its front records' lengths l =
+// q 2^-24 + r 2^-48, hi the carries out of the two words.  The window part of
+// C is summed after the window sort, where each pair's records are contiguous
+// (k_window_layout).  SLOTS as in k_mark_voxels.
+//
+// The records of 8 rows of a pixel tile share few voxels (the 64 rays are
+// neighbours).  A wave first sums runs of equal voxels along the pixel rows
+// (near the camera all 64 rays lie in one voxel, and 64 LDS operations on one
+// word follow each other: 1508 us without it), then in a table in LDS, and
+// issues one 64-bit atomic per voxel and batch: a run whose slot holds another
+// pair goes to memory by itself.  A ray meets a voxel once, so a sum in the
+// table has at most 64 parts: r < 2^30 and q < 2^31 never carry there.  In
+// memory they may (a voxel met by more than 128 rays): the add whose low word
+// wrapped takes the carry out of q again, and every carry and borrow is
+// counted in hi, modulo 2^32 per word, so the two sums stay exact.
+// 640x480 at 1 cm, 161 M records: 1125 us, of which the atomics 356; the
+// copy alone (2.6 GB) is about 600.  A copy with voxels, then a pass that
+// rewrote it in place, sorting each row's 64 pairs across the lanes, took 795
+// + 1245 us (now 1125 + 392 for k_mark_voxels, and the emission 75 more for
+// its second store).
+constexpr uint32_t kTabLog = 9, kTab = 1u << kTabLog;
+constexpr uint32_t kFree = 0xFFFFFFFFu;
+template <bool SLOTS>
+__global__ __launch_bounds__(256) void k_reslice(FrontRec* __restrict__ front, RayRec* __restrict__ lanes,
+                                                 const uint32_t* __restrict__ ids, const uint32_t* __restrict__ lens,
+                                                 const int32_t* __restrict__ slot, const uint32_t* __restrict__ pid,
+                                                 const uint32_t* __restrict__ off_f, const uint32_t* __restrict__ len_f,
+                                                 const uint32_t* __restrict__ off_w, const uint32_t* __restrict__ len_w,
+                                                 uint32_t base_w, uint2* __restrict__ inc,
+                                                 unsigned long long* __restrict__ acc,
+                                                 unsigned long long* __restrict__ hi, uint32_t* __restrict__ wkeys,
+                                                 uint32_t* __restrict__ wvals, uint32_t sentinel) {
+  constexpr uint32_t kW = 4, kB = 8;
+  __shared__ uint32_t tab_key[kW][kTab];
+  __shared__ unsigned long long tab_sum[kW][kTab];
+  const uint32_t t = blockIdx.x, wave = threadIdx.x >> 6, l = threadIdx.x & 63u, ray = t * kSlice + l;
+  uint32_t* tk = tab_key[wave];
+  unsigned long long* ts = tab_sum[wave];
+  for (uint32_t i = l; i < kTab; i += 64u) {
+    tk[i] = kFree;
+    ts[i] = 0;
+  }
+  const FrontRec f = front[ray];
+  const uint32_t rnw = lanes[ray].nw;
+  const uint32_t fo = off_f[t] + l, wo = off_w[t] + l;
+  const uint32_t lf = len_f[t], lw = len_w[t];
+  // the pairs of a batch's records (kGapVox: none)
+  auto pairs = [&](uint32_t(&e)[kB]) {
+    if constexpr (SLOTS) {
+      int32_t sl[kB];
 #pragma unroll
-    for (int j = 0; j < kR; ++j) {
-      const bool in = row0 + j < nrows;
-      e[j] = rec[(in ? row0 + j : 0) * 64 + lane];
-      if (!in) e[j].x = kGapVox;
+      for (uint32_t u = 0; u < kB; ++u) sl[u] = slot[e[u] != kGapVox ? e[u] >> kBrickLog * 3 : 0u];
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u)
+        if (e[u] != kGapVox) e[u] = (uint32_t)sl[u] * kBrickVox + (e[u] & (kBrickVox - 1u));
+    }
+    uint32_t p[kB];
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) p[u] = pid[e[u] != kGapVox ? e[u] : 0u];
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u)
+      if (e[u] != kGapVox) e[u] = p[u];
+  };
+  for (uint32_t k0 = wave * kB; k0 < lf; k0 += kW * kB) {
+    uint32_t e[kB], len[kB];
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      const bool in = k0 + u < f.nf;
+      e[u] = in ? ids[f.off + (size_t)(k0 + u) * kSlice] : kGapVox;
+      len[u] = in ? lens[f.off + (size_t)(k0 + u) * kSlice] : 0u;
+    }
+    pairs(e);
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u)
+      if (k0 + u < lf) inc[fo + (size_t)(k0 + u) * kSlice] = make_uint2(e[u], len[u]);
+    // the table: first the slots of all rows, then their sums
+    unsigned long long x[kB];
+    uint32_t at[kB], was[kB];
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      // l 2^24 is exact in double; q its integer part (< 2^25), r the rest in
+      // units of 2^-48 (< 2^24)
+      const double d = (double)__uint_as_float(len[u]) * kFixLen;
+      uint32_t q = (uint32_t)d, r = (uint32_t)((d - (double)q) * kFixLen);
+      // first summed along the pixel row: the last ray of a run of equal
+      // voxels keeps the run's sum
+      const uint32_t right = (uint32_t)__shfl_down((int)e[u], 1, 64);
+      uint32_t head = dpp_u<0x111, 0xF>(e[u]) != e[u] || (l & 7u) == 0u ? 1u : 0u;
+      const bool ends = right != e[u] || (l & 7u) == 7u;
+      seg_step_u<0x111, 0xF>(q, r, head);
+      seg_step_u<0x112, 0xF>(q, r, head);
+      seg_step_u<0x114, 0xF>(q, r, head);
+      if (!ends) e[u] = kGapVox;
+      x[u] = (unsigned long long)q << 32 | r;
+      at[u] = (e[u] * 2654435761u) >> (32 - kTabLog);
+      was[u] = e[u];
+      if (e[u] != kGapVox) was[u] = atomicCAS(&tk[at[u]], kFree, e[u]);
     }
 #pragma unroll
-    for (int j = 0; j < kR; ++j) key[j] = pid[e[j].x != kGapVox ? e[j].x : 0u];
+    for (uint32_t u = 0; u < kB; ++u)
+      if (e[u] != kGapVox && (was[u] == kFree || was[u] == e[u])) atomicAdd(&ts[at[u]], x[u]);
+    // the wave's own LDS operations complete in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int j = 0; j < kR; ++j) {
-      q[j] = r[j] = 0;
-      // every record of the row is written back (gap records unchanged), so
-      // the row's lines are written whole
-      if (row0 + j < nrows)  // uniform per row
-        rec[(row0 + j) * 64 + lane] = e[j].x != kGapVox ? make_uint2(key[j], e[j].y) : e[j];
-      if (e[j].x != kGapVox) {
-        // l 2^24 is exact in double; q its integer part (< 2^25), r the rest
-        // in units of 2^-48 (< 2^24)
-        const double x = (double)__uint_as_float(e[j].y) * kFixLen;
-        q[j] = (uint32_t)x;
-        r[j] = (uint32_t)((x - (double)q[j]) * kFixLen);
-      } else {
-        key[j] = 0xFFFFFFFFu;
-      }
-      if ((row0 + j) * 64 >= base_w) {  // a window row (uniform): the sort input only
-        if (row0 + j < nrows) {
-          const uint64_t jw = (row0 + j) * 64 - base_w + lane;
-          wkeys[jw] = key[j] == 0xFFFFFFFFu ? sentinel : key[j];
-          wvals[jw] = (uint32_t)jw;
-        }
-        key[j] = 0xFFFFFFFFu;
-        continue;
-      }
-      if constexpr (PACKED) {
-        uint32_t v = key[j] == 0xFFFFFFFFu ? 0xFFFFFFFFu : (key[j] << 6) | (uint32_t)lane;
-        sort_u32<64>(lane, v);
-        const int src = (int)(v & 63u);
-        key[j] = v == 0xFFFFFFFFu ? 0xFFFFFFFFu : v >> 6;
-        q[j] = (uint32_t)__shfl((int)q[j], src, 64);
-        r[j] = (uint32_t)__shfl((int)r[j], src, 64);
-      } else {
-        bitonic_sort<64>(lane, key[j], q[j], r[j]);
-      }
-      const uint32_t prev = (uint32_t)__shfl_up((int)key[j], 1, 64);
-      const uint32_t next = (uint32_t)__shfl_down((int)key[j], 1, 64);
-      wave_seg_sum_u(q[j], r[j], lane == 0 || prev != key[j] ? 1u : 0u);
-      // one add per run, by its last lane
-      if (!(lane == 63 || next != key[j])) key[j] = 0xFFFFFFFFu;
-    }
-    uint32_t po[kR], por[kR];
-#pragma unroll
-    for (int j = 0; j < kR; ++j) {
-      po[j] = por[j] = 0;
-      if (key[j] != 0xFFFFFFFFu) {
-        po[j] = atomicAdd(acc_f + 2 * (size_t)key[j], q[j]);
-        if (r[j]) por[j] = atomicAdd(acc_r + 2 * (size_t)key[j], r[j]);
+    for (uint32_t u = 0; u < kB; ++u) {
+      if (e[u] == kGapVox) continue;
+      if (was[u] == kFree) {  // this lane took the slot: it passes the sum on and frees the slot
+        x[u] = ts[at[u]];
+        ts[at[u]] = 0;
+        tk[at[u]] = kFree;
+      } else if (was[u] == e[u]) {
+        e[u] = kGapVox;  // in another lane's or row's sum
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // the adds, then their carries once the old values are back
+    unsigned long long old[kB];
 #pragma unroll
-    for (int j = 0; j < kR; ++j) {
-      if (key[j] == 0xFFFFFFFFu) continue;
-      if (po[j] + q[j] < po[j]) atomicAdd(acc_f + 2 * (size_t)key[j] + 1, 1u);
-      if (r[j] && por[j] + r[j] < por[j]) atomicAdd(acc_r + 2 * (size_t)key[j] + 1, 1u);
+    for (uint32_t u = 0; u < kB; ++u) old[u] = e[u] != kGapVox ? atomicAdd(acc + e[u], x[u]) : 0ull;
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      if (e[u] == kGapVox) continue;
+      unsigned long long c = old[u] + x[u] < old[u] ? 1ull << 32 : 0ull;
+      if ((uint32_t)old[u] + (uint32_t)x[u] < (uint32_t)old[u]) {
+        c += 1ull;
+        if (atomicAdd(acc + e[u], 0xFFFFFFFF00000000ull) >> 32 == 0) c -= 1ull << 32;
+      }
+      if (c) atomicAdd(hi + e[u], c);
     }
   }
+  for (uint32_t k0 = wave * kB; k0 < lw; k0 += kW * kB) {
+    uint32_t e[kB], len[kB];
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      const bool in = k0 + u < rnw;
+      e[u] = in ? ids[f.off + (size_t)(f.nf + k0 + u) * kSlice] : kGapVox;
+      len[u] = in ? lens[f.off + (size_t)(f.nf + k0 + u) * kSlice] : 0u;
+    }
+    pairs(e);
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      if (k0 + u < lw) {
+        const size_t jw = wo + (size_t)(k0 + u) * kSlice;
+        inc[base_w + jw] = make_uint2(e[u], len[u]);
+        wkeys[jw] = e[u] == kGapVox ? sentinel : e[u];
+        wvals[jw] = (uint32_t)jw;
+      }
+    }
+  }
+  __syncthreads();  // every wave has read the slice's descriptions
+  if (wave != 0) return;
+  front[ray].off = fo;
+  lanes[ray].off_w = base_w + wo;
 }
+
+// a pair's sums of q (units of 2^-24) and r (2^-48) from their words
+__device__ __forceinline__ uint64_t sum_q(uint64_t acc, uint64_t hi) { return acc >> 32 | (hi & 0xFFFFFFFF00000000ull); }
+__device__ __forceinline__ uint64_t sum_r(uint64_t acc, uint64_t hi) { return (acc & 0xFFFFFFFFull) | hi << 32; }
 
 // C in FP32 with the gate of the exact sum (C > 0.1f, gvdbkernels.cu:408) from
 // the exact fixed-point sums of a pair: w, f in units of 2^-24 (window, front
@@ -317,8 +321,8 @@ __device__ __forceinline__ float front_message(uint64_t f) { return (float)((dou
 // become the exact fixed-point parts of k_reslice; runs of equal pairs are
 // summed by a segmented scan per row of 64, a row's last run is carried into
 // the next row.  A pair whose records all lie in this tile is finished here;
-// of the others, the part in this tile is added to acc_w (units of 2^-24,
-// zeroed before) and acc_r, and k_pair_finish ends them.
+// of the others, the part in this tile is added to acc_w (units of 2^-24) and
+// acc_r (the parts below), both zeroed before, and k_pair_finish ends them.
 // Bound by its loads, so all of them are in flight before the first is used
 // (keys and indices, then the gathered records with the pairs' front sums)
 // and every store comes after the last.  640x480 at 1 cm, 30 M positions: 313
@@ -329,8 +333,10 @@ __global__ __launch_bounds__(256) void k_window_layout(const uint2* __restrict__
                                                        const uint32_t* __restrict__ win_idx, uint32_t nwin,
                                                        uint32_t nwp, uint32_t* __restrict__ wseg_off,
                                                        uint64_t* __restrict__ bits, uint32_t* __restrict__ tile_h0,
-                                                       const uint64_t* __restrict__ acc_f,
-                                                       unsigned long long* acc_w, unsigned long long* acc_r,
+                                                       const uint64_t* __restrict__ acc,
+                                                       const uint64_t* __restrict__ hi,
+                                                       unsigned long long* __restrict__ acc_w,
+                                                       unsigned long long* __restrict__ acc_r,
                                                        float* __restrict__ pair_c, float* __restrict__ pair_sf) {
   constexpr int kRows = kTile / 64;
   const int lane = threadIdx.x & 63;
@@ -355,14 +361,14 @@ __global__ __launch_bounds__(256) void k_window_layout(const uint2* __restrict__
     const uint32_t down = (uint32_t)__shfl_down((int)key[j], 1, 64);
     next[j] = lane == 63 ? after : down;
   }
-  // a run's last lane, of a pair that lies in the tile: f its front sum, r the parts below
+  // a run's last lane, of a pair that lies in the tile: its front sums
   uint64_t f[kRows], r[kRows];
 #pragma unroll
   for (int j = 0; j < kRows; ++j) {
     len[j] = key[j] != 0xFFFFFFFFu ? recw[len[j]].y : 0u;
     const bool done = key[j] != 0xFFFFFFFFu && next[j] != key[j] && key[j] != left;
-    f[j] = done ? acc_f[key[j]] : 0u;
-    r[j] = done ? acc_r[key[j]] : 0u;
+    f[j] = done ? acc[key[j]] : 0u;
+    r[j] = done ? hi[key[j]] : 0u;
   }
   uint64_t w[kRows], hb[kRows];
   uint32_t before = left;             // the key before the row
@@ -381,7 +387,9 @@ __global__ __launch_bounds__(256) void k_window_layout(const uint2* __restrict__
     const bool goes_on = (hb[j] & (~0ull >> (63 - lane))) == 0;  // still in the run from before the row
     w[j] = ql + (goes_on ? carry_w : 0u);
     const uint64_t rj = rl + (goes_on ? carry_r : 0u);
-    r[j] += rj;
+    const uint64_t fr = sum_r(f[j], r[j]) + rj;
+    f[j] = sum_q(f[j], r[j]);
+    r[j] = fr;
     before = (uint32_t)__builtin_amdgcn_readlane((int)k, 63);
     const bool carries = before == (uint32_t)__builtin_amdgcn_readlane((int)next[j], 63);
     const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)w[j], 63),
@@ -410,18 +418,19 @@ __global__ __launch_bounds__(256) void k_window_layout(const uint2* __restrict__
 
 // C and the front messages of the pairs that k_window_layout left: the
 // front-only pairs and the window pairs whose records cross a tile's end
-__global__ void k_pair_finish(const uint64_t* __restrict__ acc_w, const uint64_t* __restrict__ acc_f,
-                              const uint64_t* __restrict__ acc_r, const uint32_t* __restrict__ wseg_off, uint32_t np,
-                              uint32_t nwp, float* __restrict__ pair_c, float* __restrict__ pair_sf) {
+__global__ void k_pair_finish(const uint64_t* __restrict__ acc, const uint64_t* __restrict__ hi,
+                              const uint64_t* __restrict__ acc_w, const uint64_t* __restrict__ acc_r,
+                              const uint32_t* __restrict__ wseg_off, uint32_t np, uint32_t nwp, float* __restrict__ pair_c, float* __restrict__ pair_sf) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
-  uint64_t w = 0;
+  uint64_t w = 0, r = 0;
   if (p < nwp) {
     if (wseg_off[p] / kTile == (wseg_off[p + 1] - 1u) / kTile) return;
     w = acc_w[p];
+    r = acc_r[p];
   }
-  const uint64_t f = acc_f[p];
-  pair_c[p] = pair_length(w, f, acc_r[p]);
+  const uint64_t a = acc[p], h = hi[p], f = sum_q(a, h);
+  pair_c[p] = pair_length(w, f, sum_r(a, h) + r);
   pair_sf[p] = front_message(f);
 }
 
@@ -436,11 +445,6 @@ __global__ void k_export_vox(const uint2* __restrict__ rec, uint32_t n, const ui
 }
 
 inline unsigned blocks(size_t n, int t) { return (unsigned)((n + t - 1) / t); }
-inline unsigned stride_blocks(uint64_t n) {
-  const uint64_t b = (n + 255) / 256;
-  return (unsigned)(b < 8192 ? (b ? b : 1) : 8192);
-}
-
 }  // namespace
 
 size_t window_sort_temp_bytes(uint32_t n, int bits) {
@@ -463,33 +467,35 @@ void launch_pair_table(uint8_t* any, uint8_t* wany, const uint64_t* boff, uint32
                      pair_vox);
 }
 
-void launch_pair_lengths(uint2* rec, uint64_t nrec, uint64_t base_w, const uint32_t* pid, uint32_t* acc_f,
-                         uint32_t* acc_r, uint32_t np, uint32_t* wkeys, uint32_t* wvals, uint32_t sentinel,
-                         hipStream_t s) {
-  if (np == 0) return;
-  launch_zero_words(acc_f, (size_t)np * 8, s);
-  launch_zero_words(acc_r, (size_t)np * 8, s);
-  if (np < (1u << 26) - 1u)
-    hipLaunchKernelGGL(k_pair_lengths<true>, dim3(stride_blocks(nrec)), dim3(256), 0, s, rec, nrec, base_w, pid, acc_f,
-                       acc_r, wkeys, wvals, sentinel);
-  else
-    hipLaunchKernelGGL(k_pair_lengths<false>, dim3(stride_blocks(nrec)), dim3(256), 0, s, rec, nrec, base_w, pid,
-                       acc_f, acc_r, wkeys, wvals, sentinel);
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t nslices, const uint32_t* ids, const uint32_t* lens,
+                    const int32_t* slot, const uint32_t* pid, const uint32_t* off_f, const uint32_t* len_f,
+                    const uint32_t* off_w, const uint32_t* len_w, uint32_t base_w, uint2* inc, uint64_t* acc,
+                    uint64_t* hi, uint32_t np, uint32_t* wkeys, uint32_t* wvals, uint32_t sentinel, hipStream_t s) {
+  if (nslices == 0) return;
+  launch_zero_words(acc, (size_t)np * 8, s);
+  launch_zero_words(hi, (size_t)np * 8, s);
+  auto* k = slot ? k_reslice<true> : k_reslice<false>;
+  hipLaunchKernelGGL(k, dim3(nslices), dim3(256), 0, s, front, lanes, ids, lens, slot, pid, off_f, len_f, off_w, len_w,
+                     base_w, inc, reinterpret_cast<unsigned long long*>(acc), reinterpret_cast<unsigned long long*>(hi),
+                     wkeys, wvals, sentinel);
 }
 
 void launch_window_layout(const uint2* recw, const uint32_t* keys, const uint32_t* win_idx, uint32_t nwin,
-                          uint32_t nwp, uint32_t* wseg_off, uint64_t* bits, uint32_t* tile_h0, const uint64_t* acc_f,
-                          uint64_t* acc_w, uint64_t* acc_r, float* pair_c, float* pair_sf, hipStream_t s) {
+                          uint32_t nwp, uint32_t* wseg_off, uint64_t* bits, uint32_t* tile_h0, const uint64_t* acc,
+                          const uint64_t* hi, uint64_t* acc_w, uint64_t* acc_r, float* pair_c, float* pair_sf,
+                          hipStream_t s) {
   launch_zero_words(acc_w, (size_t)nwp * 8, s);
+  launch_zero_words(acc_r, (size_t)nwp * 8, s);
   hipLaunchKernelGGL(k_window_layout, dim3(blocks(nwin ? nwin : 1, 4 * kTile)), dim3(256), 0, s, recw, keys, win_idx,
-                     nwin, nwp, wseg_off, bits, tile_h0, acc_f, reinterpret_cast<unsigned long long*>(acc_w),
+                     nwin, nwp, wseg_off, bits, tile_h0, acc, hi, reinterpret_cast<unsigned long long*>(acc_w),
                      reinterpret_cast<unsigned long long*>(acc_r), pair_c, pair_sf);
 }
 
-void launch_pair_finish(const uint64_t* acc_w, const uint64_t* acc_f, const uint64_t* acc_r, const uint32_t* wseg_off,
-                        uint32_t np, uint32_t nwp, float* pair_c, float* pair_sf, hipStream_t s) {
+void launch_pair_finish(const uint64_t* acc, const uint64_t* hi, const uint64_t* acc_w, const uint64_t* acc_r,
+                        const uint32_t* wseg_off, uint32_t np, uint32_t nwp, float* pair_c, float* pair_sf,
+                        hipStream_t s) {
   if (np == 0) return;
-  hipLaunchKernelGGL(k_pair_finish, dim3(blocks(np, 256)), dim3(256), 0, s, acc_w, acc_f, acc_r, wseg_off, np, nwp,
+  hipLaunchKernelGGL(k_pair_finish, dim3(blocks(np, 256)), dim3(256), 0, s, acc, hi, acc_w, acc_r, wseg_off, np, nwp,
                      pair_c, pair_sf);
 }
 

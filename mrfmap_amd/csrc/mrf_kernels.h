@@ -34,7 +34,7 @@ void launch_count(const CamGeom& c, const GridGeom& g, const float* depth, const
 void launch_slice_len(const uint32_t* counts, uint32_t ntiles, uint32_t* slice_len, uint32_t* slice_rec,
                       hipStream_t s);
 // sliced-ELL emission: record k of lane l of slice t at slice_off[t] + k*64 + l
-// for k below the ray's record count (nothing past it is written), split
+// (its voxel in sell, its chord length to_len words further on) for k below the ray's record count (nothing past it is written), split
 // into front and window: front[t*64+l].nf front records, then
 // lanes[t*64+l].nw window records (the ray's description, the Kahan state of
 // the front's length sum); cnt_f / cnt_w the same per tiled pixel.  A ray
@@ -43,8 +43,8 @@ void launch_slice_len(const uint32_t* counts, uint32_t ntiles, uint32_t* slice_l
 // than 2^23 bricks in the grid): the records hold (linear brick index) * 512
 // + voxel instead of pool ids.
 void launch_emit(const CamGeom& c, const GridGeom& g, const float* depth, const float* sig, const float* bia,
-                 const int32_t* slot, const uint32_t* slice_off, const uint32_t* slice_len, uint2* sell,
-                 FrontRec* front, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_w, uint32_t* overflow,
+                 const int32_t* slot, const uint32_t* slice_off, const uint32_t* slice_len, uint32_t* sell,
+                 size_t to_len, FrontRec* front, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_w, uint32_t* overflow,
                  bool all_active, hipStream_t s);
 
 // map evaluation of one camera's pixels (log-likelihood, expected depth,
@@ -87,14 +87,17 @@ void launch_brick_flag_counts(const uint8_t* any, const uint8_t* wany, uint32_t 
 // other entries of pid are left as they are); clears any and wany behind
 void launch_pair_table(uint8_t* any, uint8_t* wany, const uint64_t* boff, uint32_t nbricks, uint32_t nwp,
                        uint32_t* pid, uint32_t* pair_vox, hipStream_t s);
-// per pair: the exact fixed-point sums of its front records' chord lengths
-// (acc_f, 2 words per pair) and of the parts below 2^-24 of its front
-// records' lengths (acc_r).  Rewrites every live record's voxel to its pair
-// (pid), and writes the window sort input: wkeys[j] = pair of window record
-// j (sentinel for a gap or padding record), wvals[j] = j.
-void launch_pair_lengths(uint2* rec, uint64_t nrec, uint64_t base_w, const uint32_t* pid, uint32_t* acc_f,
-                         uint32_t* acc_r, uint32_t np, uint32_t* wkeys, uint32_t* wvals, uint32_t sentinel,
-                         hipStream_t s);
+// copy of the staged records (voxels ids, chord lengths lens) into the final
+// front/window regions, the window region starting at base_w, each live
+// record with its pair (pid of its voxel); the window sort input: wkeys[j] =
+// pair of window record j (sentinel for a gap or padding record), wvals[j] =
+// j; and per pair the exact fixed-point sums of its front records' chord
+// lengths: acc and hi, 2 words each.  slot (may be null): the staged records
+// hold (linear brick index) * 512 + voxel and become pool ids through it
+void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t nslices, const uint32_t* ids, const uint32_t* lens,
+                    const int32_t* slot, const uint32_t* pid, const uint32_t* off_f, const uint32_t* len_f,
+                    const uint32_t* off_w, const uint32_t* len_w, uint32_t base_w, uint2* inc, uint64_t* acc,
+                    uint64_t* hi, uint32_t np, uint32_t* wkeys, uint32_t* wvals, uint32_t sentinel, hipStream_t s);
 // after the window sort (sorted pair keys and win_idx of the nwin live
 // window records), the segment layout: wseg_off[pair] = first window position
 // of the pair, wseg_off[nwp] = nwin; the bitmask of the segment heads; per
@@ -104,10 +107,12 @@ void launch_pair_lengths(uint2* rec, uint64_t nrec, uint64_t base_w, const uint3
 // leaves the sums of the others in acc_w and acc_r, launch_pair_finish ends
 // all the others
 void launch_window_layout(const uint2* recw, const uint32_t* keys, const uint32_t* win_idx, uint32_t nwin,
-                          uint32_t nwp, uint32_t* wseg_off, uint64_t* bits, uint32_t* tile_h0, const uint64_t* acc_f,
-                          uint64_t* acc_w, uint64_t* acc_r, float* pair_c, float* pair_sf, hipStream_t s);
-void launch_pair_finish(const uint64_t* acc_w, const uint64_t* acc_f, const uint64_t* acc_r, const uint32_t* wseg_off,
-                        uint32_t np, uint32_t nwp, float* pair_c, float* pair_sf, hipStream_t s);
+                          uint32_t nwp, uint32_t* wseg_off, uint64_t* bits, uint32_t* tile_h0, const uint64_t* acc,
+                          const uint64_t* hi, uint64_t* acc_w, uint64_t* acc_r, float* pair_c, float* pair_sf,
+                          hipStream_t s);
+void launch_pair_finish(const uint64_t* acc, const uint64_t* hi, const uint64_t* acc_w, const uint64_t* acc_r,
+                        const uint32_t* wseg_off, uint32_t np, uint32_t nwp, float* pair_c, float* pair_sf,
+                        hipStream_t s);
 size_t window_sort_temp_bytes(uint32_t n, int bits);
 // window region records stably sorted by pair (gap / padding records, with
 // the sentinel key, last): keys_out = pairs, vals_out = record index in the
@@ -178,22 +183,19 @@ struct CamPass {
   const uint64_t* bstart;
   const uint8_t* tail;
 };
-// copy into the final front/window regions; window region starts at base_w.
-// any / wany: pool-sized byte flags of voxels touched by a live / window
-// record (set, never cleared); counts[0] / counts[1] += the live / live
-// window records, counts[2] += all records (gap records included),
-// counts[3] += rays with records
-// slot (may be null): the staged records hold (linear brick index) * 512 +
-// voxel and become pool ids through it
+// voxels of the staged records.  any / wany: pool-sized byte flags of voxels
+// touched by a live / window record (set, never cleared); counts[0] /
+// counts[1] += the live / live window records, counts[2] += all records (gap
+// records included), counts[3] += rays with records; slot as in launch_reslice
 // bstart / tail (both or neither null), brick entries of the window records:
 // bstart[(region row of the slice) + k] bit l = record k of lane l enters a
 // brick (the ray's first record, the record after a gap, or a voxel in
 // another brick than the previous record's); tail[lane] = front records at
 // the end of the front that lie in the first window record's brick
-void launch_reslice(FrontRec* front, RayRec* lanes, uint32_t nslices, const uint2* sell, const int32_t* slot,
-                    const uint32_t* off_f, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
-                    uint32_t base_w, uint2* inc, uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail,
-                    unsigned long long* counts, hipStream_t s);
+void launch_mark_voxels(const FrontRec* front, const RayRec* lanes, uint32_t nslices, const uint32_t* ids,
+                        const int32_t* slot, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
+                        uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail, unsigned long long* counts,
+                        hipStream_t s);
 // front chunks per slice (cnt has nslices + 1 entries, the last 0), the
 // descriptor of every chunk from their offsets, and the per-lane front spans
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s);

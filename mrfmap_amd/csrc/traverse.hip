@@ -298,8 +298,9 @@ __device__ __forceinline__ Steps<F64> first_crossings(const RaySetup& rs, const 
   return st;
 }
 
-// Records of one ray are written out[0], out[kSlice], out[2 kSlice], ...
-// (record k of the 64 rays of a pixel tile is contiguous: sliced ELL), the
+// Records of one ray are written out[0], out[kSlice], out[2 kSlice], ... and
+// their chord lengths to_len words further on (record k of the 64 rays of a
+// pixel tile is contiguous: sliced ELL), the
 // first cap of them (the count goes on past cap); vis, when given, splits
 // them into front and window (vis->record(k, chord) per record in order,
 // vis->z0 the planar depth at the entry of the first).  kEmit looks each
@@ -309,8 +310,8 @@ __device__ __forceinline__ Steps<F64> first_crossings(const RaySetup& rs, const 
 // final layout turns them into pool ids.
 template <int MODE, bool F64>
 __device__ __forceinline__ WalkOut walk(const GridGeom& g, const RaySetup& rs, const Truncation& trunc,
-                                        const int32_t* __restrict__ slot, uint2* __restrict__ out, uint32_t cap,
-                                        FrontSplit* vis = nullptr) {
+                                        const int32_t* __restrict__ slot, uint32_t* __restrict__ out, size_t to_len,
+                                        uint32_t cap, FrontSplit* vis = nullptr) {
   constexpr bool kAll = MODE == kEmitAll, kWrites = MODE == kEmit || MODE == kEmitAll;
   WalkOut wo = {0u, 0.0f, true};
   Rat zin;
@@ -321,6 +322,10 @@ __device__ __forceinline__ WalkOut walk(const GridGeom& g, const RaySetup& rs, c
   double last_exit = 0.0;
   bool any = false, skipped = false;
   uint32_t cnt = 0;
+  auto put = [&](uint32_t vox, float len) {
+    out[(size_t)cnt * kSlice] = vox;
+    out[(size_t)cnt * kSlice + to_len] = __float_as_uint(len);
+  };
   // the brick's slot (kEmitAll: its linear index)
   auto brick_lookup = [&](void) -> int32_t {
     const int lin = ((ix[0] >> kBrickLog) * g.by + (ix[1] >> kBrickLog)) * g.bz + (ix[2] >> kBrickLog);
@@ -337,7 +342,7 @@ __device__ __forceinline__ WalkOut walk(const GridGeom& g, const RaySetup& rs, c
       if (!kAll && any && skipped) {
         if constexpr (kWrites) {
           float gl = (float)((zc_d - last_exit) * rs.norm);
-          if (cnt < cap) out[(size_t)cnt * kSlice] = make_uint2(kGapVox, __float_as_uint(gl));
+          if (cnt < cap) put(kGapVox, gl);
           if (vis) vis->record(cnt, gl);
         }
         ++cnt;
@@ -354,7 +359,7 @@ __device__ __forceinline__ WalkOut walk(const GridGeom& g, const RaySetup& rs, c
         const uint32_t local = (uint32_t)((((ix[0] & 7) << 3) | (ix[1] & 7)) << 3 | (ix[2] & 7));
         const uint32_t vox = (uint32_t)bslot * kBrickVox + local;
         const float len = (float)((zn_d - zc_d) * rs.norm);
-        if (cnt < cap) out[(size_t)cnt * kSlice] = make_uint2(vox, __float_as_uint(len));
+        if (cnt < cap) put(vox, len);
         if (vis) vis->record(cnt, len);
       }
       ++cnt;
@@ -578,7 +583,7 @@ __global__ void k_count(CamGeom c, GridGeom g, const float* __restrict__ depth,
   uint32_t n = 0;
   if (p.ok) {
     const Truncation trunc = truncation(g, p, sig, bia);
-    n = walk<kCount, F64>(g, p.rs, trunc, slot, nullptr, 0u).n;
+    n = walk<kCount, F64>(g, p.rs, trunc, slot, nullptr, 0, 0u).n;
   }
   counts[pix] = n;
 }
@@ -603,12 +608,13 @@ template <bool F64, bool ALL>
 __global__ void k_emit(CamGeom c, GridGeom g, const float* __restrict__ depth, const float* __restrict__ sig,
                        const float* __restrict__ bia, const int32_t* __restrict__ slot,
                        const uint32_t* __restrict__ slice_off, const uint32_t* __restrict__ slice_len,
-                       uint2* __restrict__ sell, FrontRec* __restrict__ front, RayRec* __restrict__ lanes,
+                       uint32_t* __restrict__ sell, size_t to_len, FrontRec* __restrict__ front,
+                       RayRec* __restrict__ lanes,
                        uint32_t* __restrict__ cnt_f, uint32_t* __restrict__ cnt_w, uint32_t* __restrict__ overflow) {
   const int pix = blockIdx.x * blockDim.x + threadIdx.x;
   if (pix >= tiled_pixels(c)) return;
   const uint32_t tile = (uint32_t)pix >> 6, lane = (uint32_t)pix & 63u;
-  uint2* out = sell + slice_off[tile] + lane;
+  uint32_t* out = sell + slice_off[tile] + lane;
   PixelCtx p = load_pixel(c, g, depth, pix);
   FrontRec f;
   f.off = slice_off[tile] + lane;  // front and window records follow each other until the reslice
@@ -633,7 +639,7 @@ __global__ void k_emit(CamGeom c, GridGeom g, const float* __restrict__ depth, c
     sp.open = true;
     const uint32_t cap = slice_len[tile];
     const Truncation trunc = truncation(g, p, sig, bia);
-    WalkOut wo = walk<ALL ? kEmitAll : kEmit, F64>(g, p.rs, trunc, slot, out, cap, &sp);
+    WalkOut wo = walk<ALL ? kEmitAll : kEmit, F64>(g, p.rs, trunc, slot, out, to_len, cap, &sp);
     uint32_t n = wo.n;
     if (n > cap) {  // the slot's bound did not hold: an error, and the lists stay in bounds
       atomicOr(overflow, 1u);
@@ -944,15 +950,15 @@ void launch_slice_len(const uint32_t* counts, uint32_t ntiles, uint32_t* slice_l
 }
 
 void launch_emit(const CamGeom& c, const GridGeom& g, const float* depth, const float* sig, const float* bia,
-                 const int32_t* slot, const uint32_t* slice_off, const uint32_t* slice_len, uint2* sell,
-                 FrontRec* front, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_w, uint32_t* overflow,
+                 const int32_t* slot, const uint32_t* slice_off, const uint32_t* slice_len, uint32_t* sell,
+                 size_t to_len, FrontRec* front, RayRec* lanes, uint32_t* cnt_f, uint32_t* cnt_w, uint32_t* overflow,
                  bool all_active, hipStream_t s) {
   const int n = tiled_pixels(c);
   const bool f64 = dda_fits_f64(c, g);
   auto* k = all_active ? (f64 ? k_emit<true, true> : k_emit<false, true>)
                        : (f64 ? k_emit<true, false> : k_emit<false, false>);
   hipLaunchKernelGGL(k, dim3((n + 127) / 128), dim3(128), 0, s, c, g, depth, sig, bia, slot, slice_off, slice_len, sell,
-                     front, lanes, cnt_f, cnt_w, overflow);
+                     to_len, front, lanes, cnt_f, cnt_w, overflow);
 }
 
 }  // namespace mrf
