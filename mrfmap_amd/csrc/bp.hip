@@ -1224,8 +1224,24 @@ __global__ void k_fill_f32(float* p, float v, size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_countdown(uint32_t* p) {
-  if (threadIdx.x == 0 && *p) *p -= 1u;
+// The state that the iterations of a call keep on the GPU, so that they can be
+// launched one after the other without the host: flags[0], [1] what
+// CamPass::all_pairs and msg_all point at, flags[2] the iterations so far, and
+// each iteration's residual in trace (kTraceLen entries, the last ones).
+__global__ void k_iter_begin(uint32_t* __restrict__ flags, uint64_t* __restrict__ resid) {
+  if (threadIdx.x != 0) return;
+  flags[0] = 1u;  // every pair's update
+  flags[1] = 2u;  // every pair's log2 n, two iterations
+  flags[2] = 0u;
+  *resid = 0;
+}
+__global__ void k_iter_end(uint32_t* __restrict__ flags, uint64_t* __restrict__ resid, uint64_t* __restrict__ trace) {
+  if (threadIdx.x != 0) return;
+  flags[0] = 0u;  // front-only messages are in M now
+  if (flags[1]) flags[1] -= 1u;
+  const uint32_t n = flags[2]++;
+  trace[n % kTraceLen] = *resid;
+  *resid = 0;
 }
 
 // window-touched voxels: W[v] = 1 for the voxel of every window pair
@@ -1468,7 +1484,12 @@ void launch_fill_f32(float* p, float v, size_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(n, 256)), dim3(256), 0, s, p, v, n);
 }
 
-void launch_countdown(uint32_t* p, hipStream_t s) { hipLaunchKernelGGL(k_countdown, dim3(1), dim3(64), 0, s, p); }
+void launch_iter_begin(uint32_t* flags, uint64_t* resid, hipStream_t s) {
+  hipLaunchKernelGGL(k_iter_begin, dim3(1), dim3(64), 0, s, flags, resid);
+}
+void launch_iter_end(uint32_t* flags, uint64_t* resid, uint64_t* trace, hipStream_t s) {
+  hipLaunchKernelGGL(k_iter_end, dim3(1), dim3(64), 0, s, flags, resid, trace);
+}
 
 void launch_mark_window_voxels(const uint32_t* pair_vox, uint32_t nwp, uint32_t* W, hipStream_t s) {
   if (nwp) hipLaunchKernelGGL(k_mark_window_voxels, dim3(grid_for(nwp, 256)), dim3(256), 0, s, pair_vox, nwp, W);

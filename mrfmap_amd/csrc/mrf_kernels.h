@@ -238,7 +238,12 @@ void launch_gather_pairs(const uint32_t* pair_vox, const float* dense, uint32_t 
 void launch_fill_f32(float* p, float v, size_t n, hipStream_t s);
 void launch_fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
-void launch_countdown(uint32_t* p, hipStream_t s);  // *p -= 1 unless 0
+// the start of a call and the end of an iteration: flags (3 words: all_pairs,
+// msg_all, iterations so far), the residual, which launch_iter_end moves into
+// the trace and clears
+constexpr uint32_t kTraceLen = 64;
+void launch_iter_begin(uint32_t* flags, uint64_t* resid, hipStream_t s);
+void launch_iter_end(uint32_t* flags, uint64_t* resid, uint64_t* trace, hipStream_t s);
 void launch_mark_window_voxels(const uint32_t* pair_vox, uint32_t nwp, uint32_t* W, hipStream_t s);
 void launch_dyn_flags(const uint32_t* pair_vox, uint32_t n, const uint32_t* W, uint32_t* flags, hipStream_t s);
 // the flagged indices q0 + k at dyn[pos[k]]

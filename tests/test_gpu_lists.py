@@ -50,3 +50,21 @@ def test_lists_and_marginals_match_oracle(rows, cols, focal, near, far, vis):
         np.testing.assert_array_equal(gr, orr)
         np.testing.assert_array_equal(gi, oi)
     assert np.abs(g.get_alphas().astype(np.float64) - o.alphas()).max() <= 1e-3
+
+
+@pytest.mark.parametrize("iters", [1, 64, 65, 130])
+def test_replays_without_a_wait_match_replays_with_one(iters):
+    """Without a tolerance the host waits once per 64 iterations; the residual
+    of every iteration and the marginals are those of a call that waits after
+    each (a tolerance below every residual but 0)."""
+    p, frames = _room(9, 17, 12.0, 0.1, 1.8, _lib.VIS_BRICK_LOCAL)
+    runs = []
+    for tol in (0.0, 1e-300):
+        g = gpu_for(p, frames)
+        st = g.perform_inference(max_iters=iters, tol=tol)
+        runs.append((st["iters"], g.get_trace()[0], g.get_alphas()))
+    (n0, r0, a0), (n1, r1, a1) = runs
+    assert n0 == len(r0) == iters and n1 == len(r1)
+    np.testing.assert_array_equal(r0[:n1], r1)
+    if n1 == iters:
+        np.testing.assert_array_equal(a0, a1)
