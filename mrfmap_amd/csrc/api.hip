@@ -43,6 +43,7 @@ struct Camera {
   RayRec* d_lanes = nullptr;       // one per lane of every slice (tiled pixel order)
   uint32_t* d_len_f = nullptr;     // front records per lane of each slice
   uint32_t* d_len_w = nullptr;     // window records per lane of each slice
+  uint32_t* d_order = nullptr;     // launch order of the slices in the window kernel
   bool listed = false;             // the lists below are those of the current pose and active bricks
   uint32_t nslices = 0;
   uint32_t nrays = 0;              // rays with at least one record
@@ -594,6 +595,7 @@ void free_camera_lists(Camera& cam) {
   dfree(&cam.d_lanes);
   dfree(&cam.d_len_f);
   dfree(&cam.d_len_w);
+  dfree(&cam.d_order);
   dfree(&cam.d_inc);
   dfree(&cam.d_win_idx);
   dfree(&cam.d_pair_vox);
@@ -673,6 +675,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   launch_emit(cg, c->g, cam.d_depth, c->d_sig, c->d_bia, c->d_slot, c->d_offs, c->d_has, ids, c->cap_sell0, cam.d_front,
               cam.d_lanes, c->d_counts, c->d_rayidx, overflow, all_active, s);
   if ((rc = dalloc(c, &cam.d_len_f, ntiles)) || (rc = dalloc(c, &cam.d_len_w, ntiles)) ||
+      (rc = dalloc(c, &cam.d_order, slice_order_words(ntiles))) ||
       (rc = dalloc(c, &cam.d_chunk_off, (size_t)ntiles + 1)))
     return rc;
   // ... and the front chunks, ceil(len_f / kChunk) per slice that has window
@@ -681,6 +684,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   launch_slice_len(c->d_counts, ntiles, cam.d_len_f, c->d_has, s);
   launch_exclusive_scan(c->d_has, c->d_offs, ntiles, c->d_scan_tmp, tot3, s);
   launch_slice_len(c->d_rayidx, ntiles, cam.d_len_w, c->d_counts, s);
+  launch_slice_order(cam.d_len_w, ntiles, cam.d_order, s);
   launch_exclusive_scan(c->d_counts, c->d_has, ntiles, c->d_scan_tmp, tot3 + 1, s);
   launch_chunk_counts(cam.d_len_f, cam.d_len_w, ntiles, c->d_counts, s);
   launch_exclusive_scan(c->d_counts, cam.d_chunk_off, (size_t)ntiles + 1, c->d_scan_tmp, tot3 + 2, s);
@@ -800,11 +804,11 @@ CamPass cam_pass(mrf_ctx* c, size_t ci);
 
 // Ray-kernel schedule (records loaded ahead in the front and the window
 // kernel) by size.  16 x 8 is the best or within 1 % of it from 20 k rays at
-// 4 cm to 300 k at 1 cm with up to 17 M pairs per camera (window kernel 60.9
-// us against 69.6 with 4 ahead and 62.6 with 16 for 320x240 at 2 cm, 191
-// against 207 and 195 for 640x480 at 1 cm).  With 58 M pairs per camera
+// 4 cm to 300 k at 1 cm with up to 17 M pairs per camera (window kernel 57.8
+// us against 67.1 with 4 ahead and 59.7 with 16 for 320x240 at 2 cm, 181.6
+// against 204 and 180.5 for 640x480 at 1 cm).  With 58 M pairs per camera
 // (10x10x3 m at 1 cm) the messages no longer fit the last-level cache and the
-// longer gathers want 16 ahead: 210 against 224 us.  The line is at 32 M
+// longer gathers want 16 ahead: 188 against 198 us.  The line is at 32 M
 // pairs, 128 MB of messages, half of that cache.
 int choose_schedule(const mrf_ctx* c) {
   uint32_t np = 0;
@@ -995,6 +999,7 @@ CamPass cam_pass(mrf_ctx* c, size_t ci) {
   a.lanes = cam.d_lanes;
   a.len_f = cam.d_len_f;
   a.len_w = cam.d_len_w;
+  a.order = cam.d_order;
   a.nslices = cam.nslices;
   a.inc = cam.d_inc;
   a.win_idx = cam.d_win_idx;

@@ -129,6 +129,7 @@ struct CamPass {
   const RayRec* lanes;     // one per lane of every slice
   const uint32_t* len_f;   // front records per lane of each slice
   const uint32_t* len_w;   // window records per lane of each slice
+  const uint32_t* order;   // the slice of each block of the window kernel
   uint32_t nslices;
   const uint2* inc;        // sliced records {pair | kGapVox, chord length}: front region, then window region
   const uint32_t* win_idx; // per window position (voxel order): its record's slot in the window region
@@ -201,6 +202,9 @@ void launch_mark_voxels(const FrontRec* front, const RayRec* lanes, uint32_t nsl
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s);
 void launch_chunk_desc(const uint32_t* chunk_off, const uint32_t* len_f, uint32_t nslices, uint4* desc, hipStream_t s);
 void launch_front_span(const FrontRec* front, const RayRec* lanes, uint32_t n, uint2* span, hipStream_t s);
+// the slices by descending len_w, dealt to the XCDs (slice_order_words words)
+uint32_t slice_order_words(uint32_t nslices);
+void launch_slice_order(const uint32_t* len_w, uint32_t nslices, uint32_t* order, hipStream_t s);
 // out[j] = desc[idx[j]]
 void launch_gather_desc(const uint4* desc, const uint32_t* idx, uint32_t n, uint4* out, hipStream_t s);
 void launch_pair_msgs(const CamPass& a, hipStream_t s);

@@ -24,7 +24,7 @@ def _room(rows, cols, focal, near, far, vis, seed=5):
         pose[:3, :3] = np.array([[s, 0, c], [-c, 0, s], [0, -1, 0]])
         pose[:3, 3] = (-0.9, 0.03, 0.5)
         depth = rng.uniform(near, far, (rows, cols)).astype(np.float32)
-        depth[rng.uniform(size=depth.shape) < 0.2] = 0
+        depth[rng.uniform(size=depth.shape) < (0.2 if depth.size < 100000 else 0.98)] = 0
         frames.append((pose, p.K, depth))
     return p, frames
 
@@ -35,7 +35,8 @@ def _room(rows, cols, focal, near, far, vis, seed=5):
     (8, 8, 9.0, 0.05, 0.3),    # one tile, rays of window records only and short fronts
     (9, 17, 12.0, 0.1, 1.8),   # ragged tiles, rays of every length, beyond the grid
     (40, 24, 30.0, 1.6, 1.8),  # long fronts, several batches per slice
-    (48, 48, 400.0, 0.3, 0.4), # voxels met by every ray: segments over several 512-position tiles
+    (48, 48, 400.0, 0.3, 0.4),  # voxels met by every ray: segments over several 512-position tiles
+    (744, 760, 700.0, 0.2, 1.8),  # 8835 tiles, most of few rays
 ])
 def test_lists_and_marginals_match_oracle(rows, cols, focal, near, far, vis):
     """Lists bit for bit; marginals after 2 iterations within the 1e-3 that
