@@ -713,7 +713,6 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   uint64_t* boff = bcnt + nbr;
   // (any and wany are all zero here: cleared before the first camera, and
   // behind by the pair table of each camera)
-  HIPCHK(c, hipMemsetAsync(c->d_total + 2, 0, 32, s));
   if (c->p.brick_local_vis == MRF_VIS_BRICK_LOCAL) {
     // brick entries of the window records; rows past the last slice read as
     // zero words (the window kernel's batches may look up to 16 rows past a
@@ -724,7 +723,7 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
   }
   const int32_t* brick_slot = all_active ? c->d_slot : nullptr;
   launch_mark_voxels(cam.d_front, cam.d_lanes, ntiles, ids, brick_slot, cam.d_len_f, c->d_has, cam.d_len_w, any, wany,
-                     cam.d_bstart, cam.d_tail, (unsigned long long*)(c->d_total + 2), s);
+                     cam.d_bstart, cam.d_tail, c->d_counts, c->d_total + 2, s);
   // one allocation for the partial sums, the static sums and the masks of
   // changing records (per chunk and lane each)
   const size_t nparts = (size_t)cam.nchunks * kSlice;

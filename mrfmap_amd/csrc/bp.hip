@@ -153,9 +153,10 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 // of a slice) the voxel flags any[v] = 1 (every live record) and wany[v] = 1
 // (live window records) are set, skipping a lane whose voxel equals that of
 // the ray to its left or above in the pixel tile (the flags say only
-// whether), and counts[0] / counts[1] gain the row's live / live window
-// records; counts[2] gains the slice's records (gap records included) and
-// counts[3] its rays with records.
+// whether).  counts[slice] = {live records, live window records, records
+// (gap records included), rays with records}, summed by k_slice_totals: four
+// atomics per slice on the same words took 12 ns each (240 us for 640x480
+// with few records).
 // SLOTS: the staged records hold (linear brick index) * 512 + voxel, and the
 // brick's slot is looked up here (neighbouring rays share their bricks).
 //
@@ -170,10 +171,9 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 // A block of four waves is one slice, batches of kB rows going to its waves
 // in turn: a wave's batch is a chain of loads (record, slot) before its
 // stores, and one wave per slice leaves four waves per SIMD at 640x480 and
-// fewer than one below 160x120.  640x480 at 1 cm, 161 M voxels (0.65 GB): 392
-// us, mostly the flags' byte stores; 160x120 at 4 cm: 27 us (with the copy in
-// the same pass 30, on one wave per slice and with the brick entries as a pass
-// of their own 92).
+// fewer than one below 160x120.  640x480 at 1 cm, 161 M voxels (0.65 GB): 373
+// us, mostly the flags' byte stores; with few records (2 cm, endpoint
+// activation) 28 us, and 160x120 at 4 cm 21 us.
 template <bool SLOTS>
 __global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict__ front,
                                                      const RayRec* __restrict__ lanes,
@@ -182,10 +182,9 @@ __global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict_
                                                      const uint32_t* __restrict__ off_w,
                                                      const uint32_t* __restrict__ len_w, uint8_t* __restrict__ any,
                                                      uint8_t* __restrict__ wany, uint64_t* __restrict__ bstart,
-                                                     uint8_t* __restrict__ tail,
-                                                     unsigned long long* __restrict__ counts) {
+                                                     uint8_t* __restrict__ tail, uint4* __restrict__ counts) {
   constexpr uint32_t kW = 4, kB = 8;
-  __shared__ uint64_t wave_counts[kW][2];
+  __shared__ uint32_t wave_counts[kW][2];
   const uint32_t t = blockIdx.x, wave = threadIdx.x >> 6, l = threadIdx.x & 63u, ray = t * kSlice + l;
   const FrontRec f = front[ray];
   const uint32_t rnw = lanes[ray].nw, nr = f.nf + rnw;
@@ -207,7 +206,7 @@ __global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict_
         if (e[u] != kGapVox) e[u] = (uint32_t)sl[u] * kBrickVox + (e[u] & (kBrickVox - 1u));
     }
   };
-  uint64_t nl = 0, nw = 0;
+  uint32_t nl = 0, nw = 0;  // below 2^31: the records of a camera are
   const uint32_t lf = len_f[t], lw = len_w[t];
   for (uint32_t k0 = wave * kB; k0 < lf; k0 += kW * kB) {
     uint32_t e[kB];
@@ -217,7 +216,7 @@ __global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict_
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
       const bool live = e[u] != kGapVox;
-      nl += (uint64_t)__popcll(__ballot(live));
+      nl += (uint32_t)__popcll(__ballot(live));
       const bool d = dup(e[u]);
       if (live && !d) any[e[u]] = 1;
     }
@@ -245,7 +244,7 @@ __global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict_
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
       const bool live = e[u] != kGapVox;
-      const uint64_t n = (uint64_t)__popcll(__ballot(live));
+      const uint32_t n = (uint32_t)__popcll(__ballot(live));
       nl += n;
       nw += n;
       const bool d = dup(e[u]);
@@ -283,8 +282,7 @@ __global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict_
   }
   __syncthreads();
   if (wave != 0) return;
-  // the slice's records (gap records included) and its rays with any
-  const uint64_t nray = (uint64_t)__popcll(__ballot(nr != 0u));
+  const uint32_t nray = (uint32_t)__popcll(__ballot(nr != 0u));
   uint32_t nrec = nr;
   for (int o = 32; o > 0; o >>= 1) nrec += (uint32_t)__shfl_xor((int)nrec, o, 64);
   if (l == 0) {
@@ -292,10 +290,28 @@ __global__ __launch_bounds__(256) void k_mark_voxels(const FrontRec* __restrict_
       nl += wave_counts[w][0];
       nw += wave_counts[w][1];
     }
-    if (nl) atomicAdd(&counts[0], (unsigned long long)nl);
-    if (nw) atomicAdd(&counts[1], (unsigned long long)nw);
-    if (nrec) atomicAdd(&counts[2], (unsigned long long)nrec);
-    if (nray) atomicAdd(&counts[3], (unsigned long long)nray);
+    counts[t] = make_uint4(nl, nw, nrec, nray);
+  }
+}
+
+// the sums of the slices' counts, in one block
+__global__ __launch_bounds__(1024) void k_slice_totals(const uint4* __restrict__ counts, uint32_t nslices,
+                                                       uint64_t* __restrict__ totals) {
+  __shared__ uint64_t part[16][4];
+  uint64_t s[4] = {0, 0, 0, 0};
+  for (uint32_t t = threadIdx.x; t < nslices; t += 1024u) {
+    const uint4 c = counts[t];
+    s[0] += c.x, s[1] += c.y, s[2] += c.z, s[3] += c.w;
+  }
+  for (int o = 32; o > 0; o >>= 1)
+    for (int k = 0; k < 4; ++k) s[k] += (uint64_t)__shfl_xor((unsigned long long)s[k], o, 64);
+  if ((threadIdx.x & 63u) == 0u)
+    for (int k = 0; k < 4; ++k) part[threadIdx.x >> 6][k] = s[k];
+  __syncthreads();
+  if (threadIdx.x < 4u) {
+    uint64_t v = 0;
+    for (int w = 0; w < 16; ++w) v += part[w][threadIdx.x];
+    totals[threadIdx.x] = v;
   }
 }
 
@@ -1419,12 +1435,15 @@ void launch_epilogue(const CamPass& a, hipStream_t s, int part) {
 
 void launch_mark_voxels(const FrontRec* front, const RayRec* lanes, uint32_t nslices, const uint32_t* ids,
                         const int32_t* slot, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
-                        uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail, unsigned long long* counts,
-                        hipStream_t s) {
-  if (nslices == 0) return;
-  auto* k = slot ? k_mark_voxels<true> : k_mark_voxels<false>;
-  hipLaunchKernelGGL(k, dim3(nslices), dim3(256), 0, s, front, lanes, ids, slot, len_f, off_w, len_w, any, wany, bstart,
-                     tail, counts);
+                        uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail, uint32_t* counts,
+                        uint64_t* totals, hipStream_t s) {
+  auto* c4 = reinterpret_cast<uint4*>(counts);
+  if (nslices) {
+    auto* k = slot ? k_mark_voxels<true> : k_mark_voxels<false>;
+    hipLaunchKernelGGL(k, dim3(nslices), dim3(256), 0, s, front, lanes, ids, slot, len_f, off_w, len_w, any, wany,
+                       bstart, tail, c4);
+  }
+  hipLaunchKernelGGL(k_slice_totals, dim3(1), dim3(1024), 0, s, c4, nslices, totals);
 }
 
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s) {

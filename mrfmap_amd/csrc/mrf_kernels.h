@@ -185,9 +185,10 @@ struct CamPass {
   const uint8_t* tail;
 };
 // voxels of the staged records.  any / wany: pool-sized byte flags of voxels
-// touched by a live / window record (set, never cleared); counts[0] /
-// counts[1] += the live / live window records, counts[2] += all records (gap
-// records included), counts[3] += rays with records; slot as in launch_reslice
+// touched by a live / window record (set, never cleared); totals[0..3] = the
+// live records, the live window records, all records (gap records included)
+// and the rays with records (counts: scratch, 4 words per slice); slot as in
+// launch_reslice
 // bstart / tail (both or neither null), brick entries of the window records:
 // bstart[(region row of the slice) + k] bit l = record k of lane l enters a
 // brick (the ray's first record, the record after a gap, or a voxel in
@@ -195,8 +196,8 @@ struct CamPass {
 // the end of the front that lie in the first window record's brick
 void launch_mark_voxels(const FrontRec* front, const RayRec* lanes, uint32_t nslices, const uint32_t* ids,
                         const int32_t* slot, const uint32_t* len_f, const uint32_t* off_w, const uint32_t* len_w,
-                        uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail, unsigned long long* counts,
-                        hipStream_t s);
+                        uint8_t* any, uint8_t* wany, uint64_t* bstart, uint8_t* tail, uint32_t* counts,
+                        uint64_t* totals, hipStream_t s);
 // front chunks per slice (cnt has nslices + 1 entries, the last 0), the
 // descriptor of every chunk from their offsets, and the per-lane front spans
 void launch_chunk_counts(const uint32_t* len_f, const uint32_t* len_w, uint32_t nslices, uint32_t* cnt, hipStream_t s);
