@@ -15,8 +15,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <map>
-#include <unordered_map>
 #include <chrono>
 #include <random>
 #include <cmath>
@@ -28,6 +26,7 @@
 #include <vector>
 
 #include "../../include/mrfmap_hip.h"
+#include "block_cache.h"
 #include "mrf_kernels.h"
 
 using namespace mrf;
@@ -229,36 +228,39 @@ int fail(mrf_ctx* c, int code, const std::string& msg) {
       return fail(ctx, MRF_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));             \
   } while (0)
 
-// Process-wide cache of device blocks.  A context makes some 25 allocations
-// per camera and as many frees when it is closed or a camera is traversed
-// again; hipMalloc takes 25-40 us and hipFree 80-180 us (4 x 160x120: 15 of
-// the 18 ms of a map built from nothing; 13 x 640x480: 44 of 140 ms), and for
-// lists of tens of GB the runtime takes seconds to provide the memory again
-// (a 64-keyframe build: 0.86 s in a fresh process, 4.3-4.5 s after a context
-// of that size was closed, whose frees took 2.4 s).  Blocks are therefore
-// kept on free (after the device has finished with them) and handed out again
-// for requests of up to their size and at least 4/5 of it.  Sizes below 32 MiB
-// are rounded up to eighths of a power of two, so that slightly different
-// requests share blocks; larger blocks keep their size, since lists may take
-// most of the device.  The cache keeps at most 3/4 of the device's memory, gives
-// everything back when an allocation fails, and is emptied by
-// mrf_release_device_cache(); MRF_NO_DEVICE_CACHE=1 switches it off.
-struct BlockCache {
-  std::mutex mu;
-  std::unordered_map<void*, std::pair<size_t, int>> live;  // blocks in use: bytes, device
-  std::multimap<std::pair<int, size_t>, void*> idle;        // (device, bytes) -> kept block
-  size_t kept = 0;
+// The device as the block cache (block_cache.h) sees it.  The cache keeps at
+// most 3/4 of the device's memory and is emptied by mrf_release_device_cache();
+// MRF_NO_DEVICE_CACHE=1 switches it off.
+struct HipBlocks {
+  using Error = hipError_t;
+  static int device() {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    return dev;
+  }
+  static hipError_t allocate(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+  }
+  static void release(void* p) { (void)hipFree(p); }
+  static bool wait(int dev) {
+    const int cur = device();
+    if (cur != dev) (void)hipSetDevice(dev);
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (cur != dev) (void)hipSetDevice(cur);
+    return e == hipSuccess;
+  }
+  static size_t keep_limit() {
+    size_t free_b = 0, total_b = 0;
+    return hipMemGetInfo(&free_b, &total_b) == hipSuccess ? total_b / 4 * 3 : size_t(64) << 30;
+  }
 };
 
-size_t block_size(size_t bytes) {
-  if (bytes >= size_t(32) << 20) return bytes;
-  size_t step = 512;  // 4 KiB and below: multiples of 512 B
-  while (step * 16 <= bytes) step *= 2;
-  return (bytes + step - 1) / step * step;
-}
-
-BlockCache& block_cache() {
-  static BlockCache* bc = new BlockCache;  // never destroyed: frees may run during static destruction
+BlockCache<HipBlocks>& block_cache() {
+  // never destroyed: frees may run during static destruction
+  static BlockCache<HipBlocks>* bc = new BlockCache<HipBlocks>;
   return *bc;
 }
 
@@ -270,75 +272,11 @@ bool cache_enabled() {
   return on;
 }
 
-// the cached blocks of device dev (all devices for dev < 0) back to the runtime; mu held
-void release_idle(BlockCache& bc, int dev) {
-  for (auto it = bc.idle.begin(); it != bc.idle.end();) {
-    if (dev >= 0 && it->first.first != dev) {
-      ++it;
-      continue;
-    }
-    (void)hipFree(it->second);
-    bc.kept -= it->first.second;
-    it = bc.idle.erase(it);
-  }
-}
-
 hipError_t dev_malloc(void** p, size_t bytes) {
-  *p = nullptr;
-  if (!cache_enabled()) return hipMalloc(p, bytes);
-  bytes = block_size(bytes);
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  BlockCache& bc = block_cache();
-  std::lock_guard<std::mutex> lock(bc.mu);
-  auto it = bc.idle.lower_bound({dev, bytes});
-  if (it != bc.idle.end() && it->first.first == dev && it->first.second - it->first.second / 5 <= bytes) {
-    *p = it->second;
-    bc.live[*p] = {it->first.second, dev};
-    bc.kept -= it->first.second;
-    bc.idle.erase(it);
-    return hipSuccess;
-  }
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && !bc.idle.empty()) {  // give the kept blocks back and try again
-    (void)hipGetLastError();
-    release_idle(bc, dev);
-    e = hipMalloc(p, bytes);
-  }
-  if (e == hipSuccess) bc.live[*p] = {bytes, dev};
-  return e;
+  return cache_enabled() ? block_cache().allocate(p, bytes) : HipBlocks::allocate(p, bytes);
 }
 
-void dev_free(void* p) {
-  if (!p) return;
-  BlockCache& bc = block_cache();
-  {
-    std::lock_guard<std::mutex> lock(bc.mu);
-    auto it = bc.live.find(p);
-    if (it != bc.live.end()) {
-      const size_t bytes = it->second.first;
-      const int dev = it->second.second;
-      bc.live.erase(it);
-      static size_t cap = 0;
-      if (!cap) {
-        size_t free_b = 0, total_b = 0;
-        cap = hipMemGetInfo(&free_b, &total_b) == hipSuccess ? total_b / 4 * 3 : size_t(64) << 30;
-      }
-      if (bc.kept + bytes <= cap) {
-        // the block's last uses end before another allocation can take it
-        int cur = dev;
-        (void)hipGetDevice(&cur);
-        if (cur != dev) (void)hipSetDevice(dev);
-        (void)hipDeviceSynchronize();
-        if (cur != dev) (void)hipSetDevice(cur);
-        bc.idle.insert({{dev, bytes}, p});
-        bc.kept += bytes;
-        return;
-      }
-    }
-  }
-  (void)hipFree(p);
-}
+void dev_free(void* p) { block_cache().free(p); }
 
 template <typename T>
 int dalloc(mrf_ctx* c, T** p, size_t count) {
@@ -2123,9 +2061,7 @@ int mrf_set_eval_thresholds(mrf_ctx* c, float occ_thresh, float acc_thresh) {
 }
 
 int mrf_release_device_cache(void) {
-  BlockCache& bc = block_cache();
-  std::lock_guard<std::mutex> lock(bc.mu);
-  release_idle(bc, -1);
+  (void)block_cache().give_back(-1);
   return MRF_OK;
 }
 
