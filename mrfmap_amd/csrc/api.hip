@@ -740,17 +740,27 @@ int traverse_camera(mrf_ctx* c, Camera& cam) {
 CamPass cam_pass(mrf_ctx* c, size_t ci);
 
 // Ray-kernel schedule (records loaded ahead in the front and the window
-// kernel) by size.  16 x 8 is the best or within 1 % of it from 20 k rays at
-// 4 cm to 300 k at 1 cm with up to 17 M pairs per camera (window kernel 57.8
-// us against 67.1 with 4 ahead and 59.7 with 16 for 320x240 at 2 cm, 181.6
-// against 204 and 180.5 for 640x480 at 1 cm).  With 58 M pairs per camera
-// (10x10x3 m at 1 cm) the messages no longer fit the last-level cache and the
-// longer gathers want 16 ahead: 188 against 198 us.  The line is at 32 M
-// pairs, 128 MB of messages, half of that cache.
+// kernel) by size: 16 x 8, or 16 x 16 with more than 32 M pairs in a camera,
+// except where the messages have 16 bits and the sensor model is constant.
+// 16 ahead in the window kernel takes 195 to 199 registers, so 2 waves per
+// SIMD instead of 4: as many gathers in flight from half as many rays.  That
+// pays where the messages of the rays in flight are most of the traffic and no
+// longer fit the caches.  Window kernel per camera pass with 8 and 16 ahead, us:
+//   FP32      4x4x3 m, 640x480: 16 M pairs 181 180, 31 M 206 196
+//             10x10x3 m, 640x480: 34 M 219 209, 43 M 234 221, 72 M 250 234
+//             10x10x3 m, 427x315: 35 M 124 121, 51 M 131 128
+//             10x10x3 m, 320x240: 35 M 80 82.5, 47 M 81 83
+//   16 bits   10x10x3 m, 640x480: 34 M 179 191, 60 M 194 202, 72 M 198 206
+//             10x10x3 m, 427x315: 35 M 100 112, 51 M 104 115
+//   16 bits and tables, 10x10x3 m, 640x480: 25 M 306 298, 57 M 388 368
+// Between 14 and 32 M pairs 16 ahead is up to 6 % faster for FP32 images of
+// 640x480 (12 % with tables or carried visibility) and up to 4 % slower for
+// those of 320x240.
 int choose_schedule(const mrf_ctx* c) {
   uint32_t np = 0;
   for (const Camera& cam : c->cams) np = std::max(np, cam.npairs);
-  return np > (32u << 20) ? kSchedF16W16 : kSchedF16W8;
+  const bool few_bytes = msg_bytes(msg_in_type(c->p.msg_dtype)) == 2 && c->const_model;
+  return np > (32u << 20) && !few_bytes ? kSchedF16W16 : kSchedF16W8;
 }
 
 int prepare(mrf_ctx* c) {
