@@ -819,7 +819,10 @@ __global__ __launch_bounds__(64) void k_ray_window(const RayRec* __restrict__ la
   if (lw == 0) return;
   const RayRec rec = lanes[ray];
   const uint32_t nw = rec.nw;
-  if (nw == 0) return;  // no lane-crossing operations below
+  // a lane without window records leaves: the ballots below have 0 for it, and
+  // nothing below reads a value of another lane (what is read from the first
+  // lane left, by readfirstlane, is the same in all of them)
+  if (nw == 0) return;
 
   // the front's visibility sum: the partial sums of the slice's front chunks, loaded 8 at a time
   Kahan kL = {0.f, 0.f};
@@ -1336,10 +1339,10 @@ __global__ void k_zero_u32(uint32_t* p, size_t n) {
 }
 
 inline unsigned grid_for(size_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
-// grid of the per-pair kernels: a thread per window pair, at most 4096
-// blocks strided over the front-only pairs
 // slices per XCD of the window kernel's order
 inline uint32_t order_rows(uint32_t nslices) { return (nslices + 8 * kOrderGroup - 1) / (8 * kOrderGroup) * kOrderGroup; }
+// grid of the per-pair kernels: a thread per window pair, at most 4096
+// blocks strided over the front-only pairs
 inline unsigned pair_grid(const CamPass& a) {
   return std::max(1u, std::max(grid_for(a.nwp, 256), std::min<unsigned>(grid_for(a.npairs - a.nwp, 256), 4096u)));
 }
@@ -1411,7 +1414,7 @@ void launch_epilogue(const CamPass& a, hipStream_t s, int part) {
   const float out_scale = mo == kMsgF16 ? Msg<kMsgF16>::kOut : (mo == kMsgBF16 ? Msg<kMsgBF16>::kOut : 1.0f);
   if (a.nwin && part != 2) {
     const uint32_t ntiles = (a.nwin + kTile - 1) / kTile;
-        // whole groups of blocks for the block remapping
+    // whole groups of blocks for the block remapping
     dim3 grid((grid_for(ntiles, 4) + 8 * kSegGroup - 1) / (8 * kSegGroup) * (8 * kSegGroup)), block(256);
     switch (mo) {
       case kMsgF16:

@@ -208,11 +208,17 @@ struct FrontSplit {
 // values are integers below 2^53 (dda_fits_f64): the same exact comparisons,
 // selects as fma with a factor 0 or 1, and n / d from the reciprocal of d
 // (rounded once, kept) with one residual correction.  That quotient is the
-// correctly rounded one: q + r e with e = n - d q exact has a relative error
-// below 2^-100 before its rounding, and n / d with n < 2^47 and d < 2^27 is
-// never within 2^-80 of the middle between two doubles.  Rounding keeps the
-// order, so the smallest of the three rounded crossings is the rounded
-// nearest crossing.  Steps<false> is the general form.
+// correctly rounded one.  setup_ray keeps |Oi| below 2^29 and d below 2^26, and
+// a grid has at most 2048 voxels an axis (2^27 in units of 2^-kFix), so n is
+// below 2^30.  q + r e with e = n - d q exact has a relative error below 2^-100
+// before its rounding; n / d and the middle between two doubles differ by at
+// least 1 / (d 2^54) of their value, more than 2^-80, or are equal, which would
+// take an n of 54 bits.  Rounding keeps the order, so the smallest of the three
+// rounded crossings is the rounded nearest crossing.  Steps<false> is the
+// general form.  Its quotients and those of the brick walk (mark_bricks) divide
+// the same exact doubles, so all three give the same bits, also where the tied
+// axes have other numerators: kEmitAll relies on it, since it takes every brick
+// it meets for one that the brick walk marked.
 template <bool F64>
 struct Steps;
 
