@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void k_pair_msg(const uint32_t* __restrict__ p
 // A block of four waves is one slice, batches of kB rows going to its waves
 // in turn: a wave's batch is a chain of loads (record, slot) before its
 // stores, and one wave per slice leaves four waves per SIMD at 640x480 and
-// fewer than one below 160x120.  640x480 at 1 cm, 161 M voxels (0.65 GB): 373
+// fewer than one below 160x120.  640x480 at 1 cm, 161 M voxels (0.65 GB): 362
 // us, mostly the flags' byte stores; with few records (2 cm, endpoint
 // activation) 28 us, and 160x120 at 4 cm 21 us.
 template <bool SLOTS>

@@ -150,11 +150,11 @@ __device__ __forceinline__ void wave_seg_sum_u(uint32_t& x, uint32_t& x2, uint32
 // carry and borrow is counted in hi, modulo 2^32 per word, so the two sums
 // stay exact.  The window part of C summed here as well costs 490 us more
 // (the far voxels are met by few rays of a tile) and saves 250 after the sort.
-// 640x480 at 1 cm, 161 M records: 1125 us, of which the atomics 356; the
-// copy alone (2.6 GB) is about 600.  A copy with voxels, then a pass that
-// rewrote it in place, sorting each row's 64 pairs across the lanes, took 795
-// + 1245 us (now 1125 + 392 for k_mark_voxels, and the emission 75 more for
-// its second store).
+// 640x480 at 1 cm, 150 M records in 161 M places: 1051 us and 3.87 GB by the
+// counters; the atomics take 356, the copy alone (2.6 GB) about 600.  A copy
+// with voxels, then a pass that rewrote it in place, sorting each row's 64
+// pairs across the lanes, took 795 + 1245 us (now 1051 + 362 for
+// k_mark_voxels, and the emission 75 more for its second store).
 constexpr uint32_t kTabLog = 9, kTab = 1u << kTabLog;
 constexpr uint32_t kFree = 0xFFFFFFFFu;
 template <bool SLOTS>
